@@ -83,7 +83,7 @@ size_t kv_bytes(int rows) { return (size_t)rows * QWEN_KV_WIDTH * sizeof(float);
 // ---------------------------------------------------------------------------------------------
 
 size_t decode_call_bytes(int past) {
-  return staged_layer_bytes() + decode_workspace_bytes(1) + 2 * kv_bytes(past + 1) + 4 * act_bytes(1) + 64 * 256;
+  return staged_layer_bytes() + decode_workspace_bytes(1, past + 1) + 2 * kv_bytes(past + 1) + 4 * act_bytes(1) + 64 * 256;
 }
 
 // One decode layer for one token (qwen_decode_attention_kernel.cpp:168-218 then
@@ -240,7 +240,7 @@ qwen_prefill_attention_tiles atiles(int a_seq, int a_query, int a_key, int a_hp,
 }
 
 size_t prefill_call_bytes(int S) {
-  return staged_layer_bytes() + prefill_workspace_bytes(S) + 2 * kv_bytes(S) + 4 * act_bytes(S) + 64 * 256;
+  return staged_layer_bytes() + prefill_workspace_bytes(S, 0) + 2 * kv_bytes(S) + 4 * act_bytes(S) + 64 * 256;
 }
 
 // Attention then (optionally) MLP for one prefill layer.  Host outputs: K/V rows 0..S-1, the

@@ -4,6 +4,7 @@
 // ORDERED executors (bit-exact with the reference host library) on the caller's stream.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <exception>
@@ -109,7 +110,9 @@ int qwen_hip_decode_dispatch_layers(const qwen_decode_descriptor* dsc, int n, co
     while (runnable < n && decode_descriptor_status(dsc[runnable]) == QWEN_OK) ++runnable;
     const size_t rows = runnable > 0 ? (size_t)runnable : 1u;
     rt.arena.reset();
-    rt.arena.reserve(decode_workspace_bytes(1) + 4u * QWEN_HIDDEN + 4u * rows + 512u * rows + 8192u);
+    int most = 1;  // keys of the longest history
+    for (int i = 0; i < runnable; ++i) most = std::max(most, dsc[i].past_seq_len + 1);
+    rt.arena.reserve(decode_workspace_bytes(1, most) + 4u * QWEN_HIDDEN + 4u * rows + 512u * rows + 8192u);
     std::vector<int> pasts(rows, 0);
     std::vector<float> rope_rows(rows * 128u, 0.0f);
     for (int i = 0; i < runnable; ++i) {
@@ -155,7 +158,7 @@ int qwen_hip_prefill_dispatch_layers(const qwen_prefill_descriptor* dsc, int n, 
     // a valid descriptor has at most QWEN_PREFILL_CAPACITY tokens: RoPE rows and arena sized once
     const float* rope = rt.prefill_rope(QWEN_PREFILL_CAPACITY);
     rt.arena.reset();
-    rt.arena.reserve(prefill_workspace_bytes(QWEN_PREFILL_CAPACITY) + 4096u);
+    rt.arena.reserve(prefill_workspace_bytes(QWEN_PREFILL_CAPACITY, 0) + 4096u);
     int status = QWEN_OK, done = 0;
     for (; done < n; ++done) {
       const qwen_prefill_descriptor& d = dsc[done];

@@ -9,9 +9,29 @@ namespace qwen {
 
 // ---- ORDERED (bit-exact) kernels: kernels_ordered.hip ----
 void launch_rmsnorm_ordered(const float* x, const float* w, float* y, int tokens, bool prefill, hipStream_t st);
-void launch_project_ordered(const float* x, int tokens, int in_dim, const uint8_t* W, const float* scale,
-                            const float* bias, int out_dim, float* y, const float* residual, hipStream_t st);
-void launch_silu_mul(const float* g, const float* u, float* s, size_t n, bool prefill, hipStream_t st);
+// A serial INT4 projection.  seg: the matrices whose rows the launch covers (rows 0: unused), each a
+// multiple of 64 rows, in the reference layout; y[t * stride + row].
+struct OrdSegment {
+  const uint8_t* w = nullptr;
+  const float* scale = nullptr;
+  const float* bias = nullptr;  // optional
+  float* y = nullptr;
+  int rows = 0, stride = 0;
+  int row0 = 0;                 // set by the launcher
+};
+struct OrdProject {
+  OrdSegment seg[3];
+  const float* x = nullptr;         // [tokens][in_dim], 16-byte aligned rows (any alignment with norm_w)
+  int tokens = 0, in_dim = 0;       // in_dim 1536 or 8960
+  const float* residual = nullptr;  // optional [tokens][rows]: y = residual + the chain
+  const float* norm_w = nullptr;    // x is RMS-normalized (decode) first: ordered_chain_shape only
+  int prefill = 0;                  // gate/up: the prefill SiLU
+};
+// Whether launch_project_ordered runs `rows` output rows of `tokens` tokens as chain blocks (and takes norm_w).
+bool ordered_chain_shape(int rows, int tokens);
+void launch_project_ordered(const OrdProject& a, hipStream_t st);
+// seg[0] = gate, seg[1] = up (8960 rows each): seg[0].y = SiLU(gate) * up.  norm_w: one token only.
+void launch_gate_up_ordered(const OrdProject& a, hipStream_t st);
 void launch_rope_append_decode(float* q, const float* k, const float* v, const int* pos, const float* rope,
                                bool rope_rows_are_tokens, float* k_cache, float* v_cache, size_t cache_stride,
                                int max_keys, int tokens, hipStream_t st);
@@ -21,6 +41,25 @@ void launch_rope_table_prefill(float* rope, int first, int count, hipStream_t st
 void launch_attention_ordered(const float* q, const float* k_cache, const float* v_cache, size_t cache_stride,
                               const int* pos, int max_keys, int tokens, bool prefill, int past, float* ctx,
                               hipStream_t st);
+
+// The same attention with the scores of every key kept in `scores` (attention_ordered_scores floats)
+// between its two launches.  k_new / v_new given (decode, one token): q and the new key are rotated with
+// rope and the K/V rows appended here (as launch_rope_append_decode does); otherwise q is rotated and the
+// rows are in the cache already.
+struct OrdAttentionArgs {
+  const float* q = nullptr;
+  float *k_cache = nullptr, *v_cache = nullptr;
+  size_t cache_stride = 0;
+  const int* pos = nullptr;  // decode
+  int max_keys = 0;          // prefill: past + tokens
+  bool prefill = false;
+  int past = 0;
+  const float *k_new = nullptr, *v_new = nullptr, *rope = nullptr;
+  bool rope_rows_are_tokens = false;
+  float* ctx = nullptr;
+};
+size_t attention_ordered_scores(int tokens, int max_keys);
+void launch_attention_ordered_split(const OrdAttentionArgs& a, int tokens, float* scores, hipStream_t st);
 
 // ---- FAST kernels: kernels_fast.hip ----
 constexpr int kKChunk = 128;        // K values per repacked weight chunk

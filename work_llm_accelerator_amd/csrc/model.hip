@@ -478,7 +478,7 @@ struct qwen_hip_model {
     for (int i = 0; i < count; ++i) {
       const DevLayer d = dev_layer(first + i);
       arena.reset();
-      arena.reserve(decode_workspace_bytes(B));
+      arena.reserve(decode_workspace_bytes(B, max_keys));
       DecodeBatch b{B, pos, rope_decode, false, kc0 + (size_t)i * ls, vc0 + (size_t)i * ls, (size_t)ss, max_keys};
       run_decode_attention(d, hidden, b, att, arena, stream);
       run_decode_mlp(d, att, B, hidden, arena, stream);
@@ -496,7 +496,7 @@ struct qwen_hip_model {
       for (int b = 0; b < B; ++b) {
         float* x = hidden + (size_t)b * S * QWEN_HIDDEN;
         arena.reset();
-        arena.reserve(prefill_workspace_bytes(S));
+        arena.reserve(prefill_workspace_bytes(S, past));
         run_prefill_attention(d, x, S, past, rope_prefill, kc0 + (size_t)i * ls + (size_t)b * ss,
                               vc0 + (size_t)i * ls + (size_t)b * ss, att, arena, stream);
         run_prefill_mlp(d, att, S, x, arena, stream);

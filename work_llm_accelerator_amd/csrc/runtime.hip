@@ -154,12 +154,12 @@ DevLayer stage_layer(Arena& a, const HostLayer& h, hipStream_t st) {
 
 // ---------------------------------------------------------------------------------------------
 // Executors.  Intermediates come from the arena; sizes in floats per token:
-//   xn 1536, q 1536, k 256, v 256, ctx 1536 (attention);  pn 1536, g/u/s 3*8960 (MLP).
+//   xn 1536, q 1536, k 256, v 256, ctx 1536 (attention);  pn 1536, s 8960 (MLP).
 // The attention and MLP executors each take their own part, so one token's layer needs the sum.
 namespace {
 size_t up64(size_t n) { return (n + 63u) & ~size_t(63u); }
 size_t decode_attention_floats(size_t T) { return 3u * up64(T * QWEN_HIDDEN) + 2u * up64(T * QWEN_KV_WIDTH); }
-size_t decode_mlp_floats(size_t T) { return up64(T * QWEN_HIDDEN) + 3u * up64(T * QWEN_INTERMEDIATE); }
+size_t decode_mlp_floats(size_t T) { return up64(T * QWEN_HIDDEN) + up64(T * QWEN_INTERMEDIATE); }
 
 void carve_attention_part(DecodeWorkspace& w, float* p, size_t T) {
   auto take = [&](size_t n) {
@@ -181,18 +181,19 @@ void carve_mlp_part(DecodeWorkspace& w, float* p, size_t T) {
     return r;
   };
   w.pn = take(T * QWEN_HIDDEN);
-  w.g = take(T * QWEN_INTERMEDIATE);
-  w.u = take(T * QWEN_INTERMEDIATE);
   w.s = take(T * QWEN_INTERMEDIATE);
 }
 }  // namespace
 
-// Two arena allocations (attention part, MLP part), each aligned to 256 bytes.
-size_t decode_workspace_bytes(int tokens) { return decode_workspace_floats(tokens) * sizeof(float) + 2u * 256u; }
-// run_prefill_attention's xn, q, ctx and run_prefill_mlp's pn, g, u, s: seven allocations.
-size_t prefill_workspace_bytes(int tokens) {
+// Three arena allocations (attention part, its scores, MLP part), each aligned to 256 bytes.
+size_t decode_workspace_bytes(int tokens, int max_keys) {
+  return (decode_workspace_floats(tokens) + attention_ordered_scores(tokens, max_keys)) * sizeof(float) + 3u * 256u;
+}
+// run_prefill_attention's xn, q, ctx, scores and run_prefill_mlp's pn, s: six allocations.
+size_t prefill_workspace_bytes(int tokens, int past) {
   const size_t T = (size_t)tokens;
-  return (4u * T * QWEN_HIDDEN + 3u * T * QWEN_INTERMEDIATE) * sizeof(float) + 7u * 256u;
+  return (4u * T * QWEN_HIDDEN + T * QWEN_INTERMEDIATE + attention_ordered_scores(tokens, past + tokens)) *
+             sizeof(float) + 6u * 256u;
 }
 
 size_t decode_workspace_floats(int tokens) {
@@ -207,34 +208,101 @@ DecodeWorkspace carve_decode_workspace(float* base, int tokens) {
   return w;
 }
 
+namespace {
+
+// Fused Q/K/V projection of T rows; normed: x is normalized already.
+OrdProject qkv_project(const DevLayer& L, const float* x, int T, float* q, float* k, float* v) {
+  OrdProject p;
+  p.seg[0] = OrdSegment{L.qw, L.qs, L.qb, q, QWEN_HIDDEN, QWEN_HIDDEN};
+  p.seg[1] = OrdSegment{L.kw, L.ks, L.kb, k, QWEN_KV_WIDTH, QWEN_KV_WIDTH};
+  p.seg[2] = OrdSegment{L.vw, L.vs, L.vb, v, QWEN_KV_WIDTH, QWEN_KV_WIDTH};
+  p.x = x;
+  p.tokens = T;
+  p.in_dim = QWEN_HIDDEN;
+  return p;
+}
+
+OrdProject row_project(const float* x, int T, int in_dim, const uint8_t* w, const float* scale, float* y,
+                       const float* residual) {
+  OrdProject p;
+  p.seg[0] = OrdSegment{w, scale, nullptr, y, QWEN_HIDDEN, QWEN_HIDDEN};
+  p.x = x;
+  p.tokens = T;
+  p.in_dim = in_dim;
+  p.residual = residual;
+  return p;
+}
+
+// The MLP of T rows: s = SiLU(gate) * up of the normalized rows, then out = att + down(s).
+void run_mlp(const DevLayer& L, const float* att, int T, float* out, float* pn, float* s, bool prefill,
+             hipStream_t st) {
+  OrdProject g;
+  g.seg[0] = OrdSegment{L.gw, L.gs, nullptr, s, QWEN_INTERMEDIATE, QWEN_INTERMEDIATE};
+  g.seg[1] = OrdSegment{L.uw, L.us, nullptr, nullptr, QWEN_INTERMEDIATE, QWEN_INTERMEDIATE};
+  g.tokens = T;
+  g.in_dim = QWEN_HIDDEN;
+  g.prefill = prefill ? 1 : 0;
+  if (T == 1 && !prefill) {
+    g.x = att;
+    g.norm_w = L.post_ln;
+  } else {
+    launch_rmsnorm_ordered(att, L.post_ln, pn, T, prefill, st);
+    g.x = pn;
+  }
+  launch_gate_up_ordered(g, st);
+  launch_project_ordered(row_project(s, T, QWEN_INTERMEDIATE, L.dw, L.ds, out, att), st);
+  QWEN_HIP(hipGetLastError());
+}
+
+}  // namespace
+
 void run_decode_attention_ws(const DevLayer& L, const float* x, const DecodeBatch& b, float* att,
                              const DecodeWorkspace& w, hipStream_t st) {
   const int T = b.tokens;
-  launch_rmsnorm_ordered(x, L.ln, w.xn, T, false, st);
-  launch_project_ordered(w.xn, T, QWEN_HIDDEN, L.qw, L.qs, L.qb, QWEN_HIDDEN, w.q, nullptr, st);
-  launch_project_ordered(w.xn, T, QWEN_HIDDEN, L.kw, L.ks, L.kb, QWEN_KV_WIDTH, w.k, nullptr, st);
-  launch_project_ordered(w.xn, T, QWEN_HIDDEN, L.vw, L.vs, L.vb, QWEN_KV_WIDTH, w.v, nullptr, st);
-  launch_rope_append_decode(w.q, w.k, w.v, b.pos, b.rope, b.rope_per_token, b.k_cache, b.v_cache, b.cache_stride,
-                            b.max_keys, T, st);
-  launch_attention_ordered(w.q, b.k_cache, b.v_cache, b.cache_stride, b.pos, b.max_keys, T, false, 0, w.ctx, st);
-  launch_project_ordered(w.ctx, T, QWEN_HIDDEN, L.ow, L.os, nullptr, QWEN_HIDDEN, att, nullptr, st);
+  const bool norm = ordered_chain_shape(QWEN_QKV_ROWS, T);  // the RMSNorm inside the projection's blocks
+  if (!norm) launch_rmsnorm_ordered(x, L.ln, w.xn, T, false, st);
+  OrdProject p = qkv_project(L, norm ? x : w.xn, T, w.q, w.k, w.v);
+  p.norm_w = norm ? L.ln : nullptr;
+  launch_project_ordered(p, st);
+  // One sequence rotates and appends inside the scores launch.  With several, any of them may read rows that
+  // another appends (caches that share rows), so the append is a launch before the scores.
+  const bool fuse_rope = T == 1 && w.scores;
+  if (!fuse_rope)
+    launch_rope_append_decode(w.q, w.k, w.v, b.pos, b.rope, b.rope_per_token, b.k_cache, b.v_cache, b.cache_stride,
+                              b.max_keys, T, st);
+  if (w.scores) {
+    OrdAttentionArgs a;
+    a.q = w.q;
+    a.k_cache = b.k_cache;
+    a.v_cache = b.v_cache;
+    a.cache_stride = b.cache_stride;
+    a.pos = b.pos;
+    a.max_keys = b.max_keys;
+    a.ctx = w.ctx;
+    if (fuse_rope) {
+      a.k_new = w.k;
+      a.v_new = w.v;
+      a.rope = b.rope;
+      a.rope_rows_are_tokens = b.rope_per_token;
+    }
+    launch_attention_ordered_split(a, T, w.scores, st);
+  } else {
+    launch_attention_ordered(w.q, b.k_cache, b.v_cache, b.cache_stride, b.pos, b.max_keys, T, false, 0, w.ctx, st);
+  }
+  launch_project_ordered(row_project(w.ctx, T, QWEN_HIDDEN, L.ow, L.os, att, nullptr), st);
   QWEN_HIP(hipGetLastError());
 }
 
 void run_decode_mlp_ws(const DevLayer& L, const float* att, int T, float* out, const DecodeWorkspace& w,
                        hipStream_t st) {
-  launch_rmsnorm_ordered(att, L.post_ln, w.pn, T, false, st);
-  launch_project_ordered(w.pn, T, QWEN_HIDDEN, L.gw, L.gs, nullptr, QWEN_INTERMEDIATE, w.g, nullptr, st);
-  launch_project_ordered(w.pn, T, QWEN_HIDDEN, L.uw, L.us, nullptr, QWEN_INTERMEDIATE, w.u, nullptr, st);
-  launch_silu_mul(w.g, w.u, w.s, (size_t)T * QWEN_INTERMEDIATE, false, st);
-  launch_project_ordered(w.s, T, QWEN_INTERMEDIATE, L.dw, L.ds, nullptr, QWEN_HIDDEN, out, att, st);
-  QWEN_HIP(hipGetLastError());
+  run_mlp(L, att, T, out, w.pn, w.s, false, st);
 }
 
 void run_decode_attention(const DevLayer& L, const float* x, const DecodeBatch& b, float* att, Arena& a,
                           hipStream_t st) {
   DecodeWorkspace w{};
   carve_attention_part(w, a.alloc_n<float>(decode_attention_floats((size_t)b.tokens)), (size_t)b.tokens);
+  w.scores = a.alloc_n<float>(attention_ordered_scores(b.tokens, b.max_keys));
   run_decode_attention_ws(L, x, b, att, w, st);
 }
 
@@ -251,27 +319,27 @@ void run_prefill_attention(const DevLayer& L, const float* x, int T, int past, c
   float* xn = a.alloc_n<float>((size_t)T * QWEN_HIDDEN);
   float* q = a.alloc_n<float>((size_t)T * QWEN_HIDDEN);
   float* ctx = a.alloc_n<float>((size_t)T * QWEN_HIDDEN);
+  float* scores = a.alloc_n<float>(attention_ordered_scores(T, past + T));
   launch_rmsnorm_ordered(x, L.ln, xn, T, true, st);
-  launch_project_ordered(xn, T, QWEN_HIDDEN, L.kw, L.ks, L.kb, QWEN_KV_WIDTH, k_new, nullptr, st);
-  launch_project_ordered(xn, T, QWEN_HIDDEN, L.vw, L.vs, L.vb, QWEN_KV_WIDTH, v_new, nullptr, st);
-  launch_project_ordered(xn, T, QWEN_HIDDEN, L.qw, L.qs, L.qb, QWEN_HIDDEN, q, nullptr, st);
+  launch_project_ordered(qkv_project(L, xn, T, q, k_new, v_new), st);
   launch_rope_prefill(q, k_new, rope + (size_t)past * 128, T, st);
-  launch_attention_ordered(q, k_rows, v_rows, 0, nullptr, past + T, T, true, past, ctx, st);
-  launch_project_ordered(ctx, T, QWEN_HIDDEN, L.ow, L.os, nullptr, QWEN_HIDDEN, att, nullptr, st);
+  OrdAttentionArgs args;
+  args.q = q;
+  args.k_cache = k_rows;
+  args.v_cache = v_rows;
+  args.max_keys = past + T;
+  args.prefill = true;
+  args.past = past;
+  args.ctx = ctx;
+  launch_attention_ordered_split(args, T, scores, st);
+  launch_project_ordered(row_project(ctx, T, QWEN_HIDDEN, L.ow, L.os, att, nullptr), st);
   QWEN_HIP(hipGetLastError());
 }
 
 void run_prefill_mlp(const DevLayer& L, const float* att, int T, float* out, Arena& a, hipStream_t st) {
   float* pn = a.alloc_n<float>((size_t)T * QWEN_HIDDEN);
-  float* g = a.alloc_n<float>((size_t)T * QWEN_INTERMEDIATE);
-  float* u = a.alloc_n<float>((size_t)T * QWEN_INTERMEDIATE);
   float* s = a.alloc_n<float>((size_t)T * QWEN_INTERMEDIATE);
-  launch_rmsnorm_ordered(att, L.post_ln, pn, T, true, st);
-  launch_project_ordered(pn, T, QWEN_HIDDEN, L.gw, L.gs, nullptr, QWEN_INTERMEDIATE, g, nullptr, st);
-  launch_project_ordered(pn, T, QWEN_HIDDEN, L.uw, L.us, nullptr, QWEN_INTERMEDIATE, u, nullptr, st);
-  launch_silu_mul(g, u, s, (size_t)T * QWEN_INTERMEDIATE, true, st);
-  launch_project_ordered(s, T, QWEN_INTERMEDIATE, L.dw, L.ds, nullptr, QWEN_HIDDEN, out, att, st);
-  QWEN_HIP(hipGetLastError());
+  run_mlp(L, att, T, out, pn, s, true, st);
 }
 
 }  // namespace qwen

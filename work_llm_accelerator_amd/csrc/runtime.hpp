@@ -120,9 +120,9 @@ struct DecodeBatch {
   int max_keys;            // cache rows per sequence the caller sized (key counts are clamped to it)
 };
 
-// Arena bytes the executors below need for `tokens` tokens.
-size_t decode_workspace_bytes(int tokens);
-size_t prefill_workspace_bytes(int tokens);
+// Arena bytes the executors below need for `tokens` tokens (decode: max_keys as in DecodeBatch).
+size_t decode_workspace_bytes(int tokens, int max_keys);
+size_t prefill_workspace_bytes(int tokens, int past);
 
 void run_decode_attention(const DevLayer& L, const float* x, const DecodeBatch& b, float* att, Arena& a,
                           hipStream_t st);
@@ -130,9 +130,11 @@ void run_decode_mlp(const DevLayer& L, const float* att, int tokens, float* out,
 
 // The same executors over caller-provided intermediates (device memory of `tokens` rows each):
 // attention xn, q [tokens][1536], k, v [tokens][256], ctx [tokens][1536]; MLP pn [tokens][1536],
-// g, u, s [tokens][8960].
+// s [tokens][8960].  scores (attention_ordered_scores floats) is not part of the carve-up: its size
+// follows the key count, and without it (null) the attention runs as one launch that keeps no scores.
 struct DecodeWorkspace {
-  float *xn, *q, *k, *v, *ctx, *pn, *g, *u, *s;
+  float *xn, *q, *k, *v, *ctx, *pn, *s;
+  float* scores = nullptr;
 };
 // Floats of a DecodeWorkspace of `tokens` rows, and its carve-up of `base` (each part 64-float aligned).
 size_t decode_workspace_floats(int tokens);
