@@ -187,6 +187,91 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) l
   }
 }
 
+// 17 and more tokens: the table streamed once for NT token tiles (lm_head_kernel reads it once per tile).
+// 256 blocks of 8 waves, one per CU, each with its NT * 16 normalized rows in LDS (49 KB per tile, so up to
+// three tiles); wave w of the grid takes the 16-row table tiles w, w + waves, ..., eight 16-byte K steps per
+// lane in flight across the tile boundaries.  Bound by HBM: with the norm launch, 24 tokens x 151936
+// rows 213 -> 113 us, 48 tokens 317 -> 126 us, 64 tokens (two passes of two tiles) 424 -> 234 us.
+// The sums run in lm_head_kernel's K order, so the logits are the same bits.
+template <bool LOGITS, int NT>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
+lm_head_stream_kernel(const uint16_t* __restrict__ table, int vocab, const uint16_t* __restrict__ xn, int first, int count,
+                      float* __restrict__ logits, unsigned long long* __restrict__ best) {
+  __shared__ __align__(16) uint16_t xs[NT * 16 * kHeadRow];
+  __shared__ unsigned long long red[8][NT * 16];
+  constexpr int kSteps = QWEN_HIDDEN / 32, kAhead = 8;
+  static_assert(kSteps % kAhead == 0, "whole rings of K steps");
+  const int live_rows = min(NT * 16, count - first);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, g = lane >> 4;
+  const int ntiles = vocab / 16, stride = gridDim.x * 8;
+  int tile = blockIdx.x * 8 + wave;
+  auto tile_ptr = [&](int t) {  // tiles past the last reload it (not used)
+    return reinterpret_cast<const hf32x4*>(table + (size_t)(min(t, ntiles - 1) * 16 + col) * QWEN_HIDDEN) + g;
+  };
+  const hf32x4* ap = tile_ptr(tile);
+  hf32x4 a[kAhead];
+#pragma unroll
+  for (int s = 0; s < kAhead; ++s) a[s] = __builtin_nontemporal_load(ap + 4 * s);
+  for (int i = threadIdx.x; i < live_rows * (QWEN_HIDDEN / 8); i += 512) {
+    const int r = i / (QWEN_HIDDEN / 8), c = i % (QWEN_HIDDEN / 8);
+    *reinterpret_cast<uint4*>(xs + r * kHeadRow + 8 * c) =
+        *reinterpret_cast<const uint4*>(xn + (size_t)(first + r) * QWEN_HIDDEN + 8 * c);
+  }
+  __syncthreads();
+  const uint16_t* xrow[NT];  // columns past the last token read row 0 (not stored)
+#pragma unroll
+  for (int n = 0; n < NT; ++n) xrow[n] = xs + (n * 16 + col < live_rows ? n * 16 + col : 0) * kHeadRow + 8 * g;
+  unsigned long long bk[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) bk[n] = 0ull;
+  for (; tile < ntiles; tile += stride) {
+    const hf32x4* next = tile_ptr(tile + stride);
+    hf32x4 acc[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[n] = hf32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1  // (unrolled, the compiler reads every step's tokens ahead and spills)
+    for (int kb = 0; kb < kSteps / kAhead; ++kb) {
+      const hf32x4* load = kb + 1 < kSteps / kAhead ? ap + 4 * kAhead * (kb + 1) : next;
+#pragma unroll
+      for (int s = 0; s < kAhead; ++s) {
+        hbf16x8 av;
+        __builtin_memcpy(&av, &a[s], 16);
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+          acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              av, *reinterpret_cast<const hbf16x8*>(xrow[n] + 32 * (kb * kAhead + s)), acc[n], 0, 0, 0);
+        a[s] = __builtin_nontemporal_load(load + 4 * s);
+      }
+    }
+    ap = next;
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      float lf[4];
+      const unsigned long long key = head_best(acc[n], tile * 16, g, lf);
+      bk[n] = key > bk[n] ? key : bk[n];
+      const int tok = first + n * 16 + col;
+      if (LOGITS && tok < count)
+        *reinterpret_cast<float4*>(logits + (size_t)tok * vocab + tile * 16 + 4 * g) = make_float4(lf[0], lf[1], lf[2], lf[3]);
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+#pragma unroll
+    for (int off = 16; off < 64; off <<= 1) {
+      const unsigned long long o = __shfl_xor(bk[n], off, 64);
+      bk[n] = o > bk[n] ? o : bk[n];
+    }
+    if (g == 0) red[wave][n * 16 + col] = bk[n];
+  }
+  __syncthreads();
+  if (threadIdx.x < NT * 16 && first + (int)threadIdx.x < count) {
+    unsigned long long m = red[0][threadIdx.x];
+#pragma unroll
+    for (int w = 1; w < 8; ++w) m = red[w][threadIdx.x] > m ? red[w][threadIdx.x] : m;
+    best[(size_t)(first + threadIdx.x) * gridDim.x + blockIdx.x] = m;
+  }
+}
+
 // One token (greedy decode): each logit as a dot product on the VALU, so that every load reads 1 KiB of
 // one table row (lm_head_kernel's MFMA A operand reads 64 B of 16 rows per load: 5.0 TB/s).  grid =
 // vocab / 128, block = 256; wave w of block vb takes rows vb*128 + 32w .. + 31, two at a time with the
@@ -327,6 +412,34 @@ __global__ void __launch_bounds__(256) argmax_finalize_kernel(const unsigned lon
   }
 }
 
+namespace {
+
+constexpr int kHeadStreamFrom = 16;  // more tokens than this: lm_head_stream_kernel
+
+template <bool LOGITS, int NT>
+void launch_head_stream(const uint16_t* table, int vocab, const uint16_t* xn, int first, int count, int blocks,
+                        float* logits, unsigned long long* best, hipStream_t st) {
+  hipLaunchKernelGGL((lm_head_stream_kernel<LOGITS, NT>), dim3(blocks), dim3(512), 0, st, table, vocab, xn, first, count,
+                     logits, best);
+}
+
+// `count` tokens in passes of at most three token tiles, as even as the tiles allow.
+template <bool LOGITS>
+void launch_head_stream_all(const uint16_t* table, int vocab, const uint16_t* xn, int count, int blocks, float* logits,
+                            unsigned long long* best, hipStream_t st) {
+  const int tiles = (count + 15) / 16, passes = (tiles + 2) / 3, per = (tiles + passes - 1) / passes;
+  for (int t = 0; t < tiles; t += per) {
+    if (per == 1)
+      launch_head_stream<LOGITS, 1>(table, vocab, xn, t * 16, count, blocks, logits, best, st);
+    else if (per == 2)
+      launch_head_stream<LOGITS, 2>(table, vocab, xn, t * 16, count, blocks, logits, best, st);
+    else
+      launch_head_stream<LOGITS, 3>(table, vocab, xn, t * 16, count, blocks, logits, best, st);
+  }
+}
+
+}  // namespace
+
 size_t head_workspace_bytes(int count, int vocab) {
   const size_t rows = (size_t)((count + 15) / 16) * 16;
   return rows * QWEN_HIDDEN * 2u + (size_t)count * (size_t)(vocab / (2 * kHeadBlockRows)) * 8u + 256u;
@@ -339,7 +452,7 @@ void launch_head(const float* hidden, int count, const uint16_t* norm_w, const u
   const size_t xn_bytes = (size_t)tiles * 16 * QWEN_HIDDEN * 2u;
   unsigned long long* best =
       reinterpret_cast<unsigned long long*>(static_cast<char*>(workspace) + ((xn_bytes + 255u) & ~size_t(255u)));
-  const int nblk = vocab / (2 * kHeadBlockRows);
+  int nblk = vocab / (2 * kHeadBlockRows);  // blocks with a best key per token
   const size_t lds = (size_t)(count < 16 ? count : 16) * kHeadRow * 2u;  // live token rows of a tile
   // one token: the norm runs inside every lm_head block (no launch of its own)
   if (count == 1 && logits)
@@ -350,7 +463,13 @@ void launch_head(const float* hidden, int count, const uint16_t* norm_w, const u
                        hidden, norm_w);
   else {
     hipLaunchKernelGGL(head_norm_kernel, dim3(tiles * 16), dim3(256), 0, st, hidden, count, norm_w, xn);
-    if (logits)
+    if (count > kHeadStreamFrom) {
+      if (nblk > 256) nblk = 256;
+      if (logits)
+        launch_head_stream_all<true>(table, vocab, xn, count, nblk, logits, best, st);
+      else
+        launch_head_stream_all<false>(table, vocab, xn, count, nblk, logits, best, st);
+    } else if (logits)
       hipLaunchKernelGGL(lm_head_kernel<true>, dim3(nblk, tiles), dim3(256), lds, st, table, vocab, xn, count, logits,
                          best);
     else
