@@ -72,7 +72,7 @@ constexpr int kEpiStore = 0, kEpiSiluMul = 1, kEpiResidual = 2;
 //   kFuseQkvRope:   [q|k|v] rows + bias, decode RoPE of q and k, K/V cache append (kEpiStore);
 //   kFuseNormQuant: the finished row (kEpiStore, or kEpiResidual after bf16 rounding) is RMS-normalized
 //                   with norm_w and quantized into xq_out / sx_out / sums_out for the next projection.
-// Fused into the epilogue of the pipelined GEMM (more than kSplitTokens tokens):
+// Fused into the epilogue of the pipelined GEMM (more than kSkinnyTokens tokens):
 //   kFuseRopePrefill: [q|k|v] rows + bias, prefill RoPE of q (in place in y) and k, K/V cache append;
 //                     token t is sequence t / seq_len at position past + t % seq_len.
 constexpr int kFuseNone = 0, kFuseQkvRope = 1, kFuseNormQuant = 2, kFuseRopePrefill = 3;
@@ -125,7 +125,7 @@ struct GemmArgs {
   int round_bf16;       // kEpiResidual: round the output to bf16 (driver rounding)
   int prefill_silu;     // kEpiSiluMul: 1 = approx_exp SiLU (prefill), 0 = expf SiLU (decode)
   float* part;          // optional fp32 workspace for K splits across blocks: [splits][tokens][out]
-  int fuse;             // kFuse*: epilogue of the reduce kernel (needs part; tokens <= kSplitTokens)
+  int fuse;             // kFuse*: epilogue of the reduce kernel (needs part)
   // kFuseQkvRope (token t is sequence t at position pos[t]; positions outside [0, limit) are skipped)
   const int* pos;
   const float* rope;    // [position][cos 64 | sin 64]
@@ -159,10 +159,13 @@ struct GemmArgs {
   int amax_n;
 };
 
-// K splits across blocks: at most kMaxSplits splits, only for GEMMs of at most kSplitTokens tokens;
-// the workspace holds kMaxSplits x kSplitTokens x out floats.
+// K splits across blocks: at most kMaxSplits splits and kSplitRows rows (splits x tokens) of partials;
+// the workspace holds kSplitRows x out floats.  kSplitTokens: the largest decode batch whose reduce steps
+// carry the fused epilogues; kPrefillFuseTokens: the same for the RMSNorm + quantization of a prefill.
 constexpr int kMaxSplits = 16;
 constexpr int kSplitTokens = 256;
+constexpr int kSplitRows = 8192;
+constexpr int kPrefillFuseTokens = 1024;
 // K splits of the one-token down projection (8960 = 5 x 14 chunks of 128), whose partials the next
 // layer's Q/K/V blocks reduce in their prologue.
 constexpr int kPreResidualSplits = 5;
@@ -172,7 +175,7 @@ constexpr int kPreResidualSplits = 5;
 constexpr int kOneTokenOSplits = 2;
 // Decode GEMMs of at most kSkinnyTokens tokens (in_dim 1536 or 8960) run the skinny kernels.
 constexpr int kSkinnyTokens = 64;
-inline size_t splitk_bytes(size_t out) { return (size_t)kMaxSplits * kSplitTokens * out * 4u; }
+inline size_t splitk_bytes(size_t out) { return (size_t)kSplitRows * out * 4u; }
 
 void launch_repack_int4(const uint8_t* W, int out_dim, int in_dim, uint8_t* WP, hipStream_t st);
 void launch_norm_quant(const float* x, size_t x_stride, int rows, int n, const float* w, int norm, int8_t* xq,
@@ -228,11 +231,18 @@ void launch_attn_decode(const float* qkv, int qkv_stride, const float* k_cache, 
                         float* part, float2* pml, float* ctx, int8_t* xq, float* sx, int* sums, hipStream_t st);
 // Prefill attention of S new tokens per sequence at positions past..past+S-1 over the cache rows
 // 0..past+S-1: K/V converted once into bf16 hi/lo tiles (workspace of
-// attn_prefill_workspace_bytes(past + S, nseq)), then the causal attention over them.
+// attn_prefill_workspace_bytes(past + S, nseq)), then the causal attention over them into ctx.  The plan
+// splits the key tiles of a query tile over nsplit blocks of tps tiles where the query tiles alone leave the
+// device idle (workspace: part [nseq*S][12][nsplit][128], pml [nseq*S][12][nsplit]): the merge of the splits
+// then also forms the O projection's input code (xq, sx, sums), and ctx is not written.
+struct AttnPrefillPlan {
+  int nsplit, tps;
+};
+AttnPrefillPlan plan_attn_prefill(int S, int past, int nseq);
 size_t attn_prefill_workspace_bytes(int keys, int nseq);
 void launch_attn_prefill(const float* qkv, int qkv_stride, const float* k_cache, const float* v_cache,
-                         size_t seq_stride, int S, int past, int nseq, uint8_t* kv_tiles, float* ctx,
-                         hipStream_t st);
+                         size_t seq_stride, int S, int past, int nseq, uint8_t* kv_tiles, const AttnPrefillPlan& plan,
+                         float* part, float2* pml, float* ctx, int8_t* xq, float* sx, int* sums, hipStream_t st);
 void launch_round_bf16(float* x, size_t n, hipStream_t st);
 
 }  // namespace qwen

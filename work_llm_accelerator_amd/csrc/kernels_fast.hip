@@ -708,15 +708,16 @@ constexpr int kIntSumMaxK = 8192;
 // its accumulator slot 0, and the wave runs half of that slot's MFMAs before the chunk's barrier (its
 // own loads have landed by its own wait), so waves that reach the barrier late are absorbed by matrix
 // work instead of stalling the others.  Slot n holds token tile (wv + n) mod 4.
-// ROPE (the fused [q | k | v] projection of a prefill, kFuseRopePrefill): wave w of a block (2 heads,
+// ROPE (the fused [q | k | v] projection of a prefill, kFuseRopePrefill): wave w of a block (RTW = 4: 2 heads,
 // 16 row tiles) holds row tiles h*8 + 2*(w & 1) + {0, 1} and the same + 4 of head h = w >> 1, so that
 // tiles r and r + 2 hold the rotation pairs (p, p + 64) of one head and the epilogue rotates q and k and
-// appends K/V to the cache, as rope_qkv_kernel does after a plain store.
+// appends K/V to the cache, as rope_qkv_kernel does after a plain store.  RTW = 2 (one head per block, for
+// launches whose 2-head blocks would leave CUs idle): wave w holds row tiles w and w + 4 of its head.
 template <int NT, int RTW, int NBUF, int EPI, bool DUAL, int TW, int WPE = 1, bool OWN = false, bool ROPE = false,
           int EF = 0>
 __global__ void __launch_bounds__(256 * TW) __attribute__((amdgpu_waves_per_eu(WPE))) gemm_i8_pipe_kernel(GemmArgs a) {
   static_assert(!OWN || (TW == 1 && NT == 4), "own tile first: each of the 4 waves loads one token tile");
-  static_assert(!ROPE || (RTW == 4 && TW == 1 && !DUAL && EPI == kEpiStore), "prefill RoPE: 2 heads per block");
+  static_assert(!ROPE || ((RTW == 4 || RTW == 2) && TW == 1 && !DUAL && EPI == kEpiStore), "prefill RoPE: 1 or 2 heads per block");
   constexpr int D = DUAL ? 2 : 1;
   constexpr int TOK = 16 * NT * TW;        // tokens per block (TW token groups of 16*NT)
   constexpr int XB = TOK * 256;                 // activation bytes per stage
@@ -761,6 +762,7 @@ __global__ void __launch_bounds__(256 * TW) __attribute__((amdgpu_waves_per_eu(W
   const int rt0 = ((within / gsize) * 4 + wave) * RTW;  // the wave's first row tile
   // row tile of the wave's tile r
   auto row_tile = [&](int r) {
+    if (ROPE && RTW == 2) return (within / gsize) * 8 + wave + r * 4;
     return ROPE ? (within / gsize) * 16 + (wave >> 1) * 8 + (wave & 1) * 2 + (r & 1) + (r >> 1) * 4 : rt0 + r;
   };
   const int tok0 = (first_t + within % gsize) * TOK;   // the block's first token
@@ -923,10 +925,11 @@ __global__ void __launch_bounds__(256 * TW) __attribute__((amdgpu_waves_per_eu(W
       }
     }
     if constexpr (ROPE) {
-      // tiles r and r + 2 (r < 2): dims p .. p + 3 and p + 64 .. p + 67 of head rt / 8; cos/sin of the
+      // tiles r and r + RTW / 2: dims p .. p + 3 and p + 64 .. p + 67 of head rt / 8; cos/sin of the
       // lane's tokens are loaded per pair, so that one pair's 32 registers are live at a time
+      constexpr int HR = RTW / 2;
 #pragma unroll
-      for (int r = 0; r < 2; ++r) {
+      for (int r = 0; r < HR; ++r) {
         const int rt = row_tile(r);
         const int head = rt >> 3;
         const int p = (rt & 7) * 16 + 4 * g;
@@ -949,8 +952,8 @@ __global__ void __launch_bounds__(256 * TW) __attribute__((amdgpu_waves_per_eu(W
           for (int q = 0; q < 4; ++q) {
             e[q] = (float)(accH[0][r][n][q] - sh8[n]) * 256.0f + (float)(accL[0][r][n][q] - sl8[n]);
             e[q] = e[q] * sxv[n] * sw[r][q] + bias[r][q];
-            od[q] = (float)(accH[0][r + 2][n][q] - sh8[n]) * 256.0f + (float)(accL[0][r + 2][n][q] - sl8[n]);
-            od[q] = od[q] * sxv[n] * sw[r + 2][q] + bias[r + 2][q];
+            od[q] = (float)(accH[0][r + HR][n][q] - sh8[n]) * 256.0f + (float)(accL[0][r + HR][n][q] - sl8[n]);
+            od[q] = od[q] * sxv[n] * sw[r + HR][q] + bias[r + HR][q];
           }
           const float c4[4] = {cs[n].x, cs[n].y, cs[n].z, cs[n].w}, s4[4] = {sn[n].x, sn[n].y, sn[n].z, sn[n].w};
           float lo[4], hi[4];
@@ -3346,7 +3349,8 @@ attn_decode_kernel(const float* __restrict__ qkv, int qkv_stride, const float* _
   }
 }
 
-// The split merge of attn_decode_kernel's partials, one block per sequence: per head the merge
+// The split merge of attn_decode_kernel's partials, one block per sequence (pos given), or of the split prefill
+// attention's, one block per token (pos null: token b at position past + b % seq_len): per head the merge
 // weights of the splits that hold keys (merge_split_weights), the weighted sum of their partial rows
 // in split order into the context row (written to ctx when given), then the row's two-limb code,
 // scale and limb sums for the O projection (quantize_row_lds).  Thread t owns float4 columns t and
@@ -3355,8 +3359,9 @@ attn_decode_kernel(const float* __restrict__ qkv, int qkv_stride, const float* _
 // at most 8 splits need one memory round trip.
 __global__ void __launch_bounds__(256) attn_decode_merge_kernel(const float* __restrict__ part,
                                                                 const float2* __restrict__ pml,
-                                                                const int* __restrict__ pos, int nsplit, int chunk,
-                                                                int max_keys, float* __restrict__ ctx,
+                                                                const int* __restrict__ pos, int seq_len, int past,
+                                                                int nsplit, int chunk, int max_keys,
+                                                                float* __restrict__ ctx,
                                                                 int8_t* __restrict__ xq, float* __restrict__ sx,
                                                                 int* __restrict__ sums) {
   constexpr int kF4 = QWEN_HIDDEN / 4;  // float4 columns of the row
@@ -3365,7 +3370,7 @@ __global__ void __launch_bounds__(256) attn_decode_merge_kernel(const float* __r
   __shared__ float red_f[4];
   __shared__ int red_i[8];
   const int b = blockIdx.x;
-  const int n = min(max(pos[b], 0) + 1, max_keys);
+  const int n = pos ? min(max(pos[b], 0) + 1, max_keys) : past + b % seq_len + 1;
   const int nc = (n + chunk - 1) / chunk;  // splits that hold keys
   const float2* pb = pml + (size_t)b * QWEN_Q_HEADS * nsplit;
   const float* pa = part + (size_t)b * QWEN_Q_HEADS * nsplit * QWEN_HEAD_DIM;
@@ -3525,26 +3530,38 @@ __global__ void __launch_bounds__(256) kv_bf16_tiles_kernel(const float* __restr
 // blocks share each CU and their phases interleave.  Measured at 8 x 2048 against one 14-wave block
 // of 32 queries with a 3-stage ring per CU: 410 -> 362 us, bit-identical.
 // grid = (ceil(S/16), 2, nseq) with query tiles longest first, block = 448.
+// SPLIT: few query tiles leave most CUs idle, so the key tiles of a query tile go to several blocks of tps
+// tiles each (grid.z = nseq * nsplit); a block leaves its queries' unnormalized rows and (max, sum) in
+// part[token][head][split][128], pml[token][head][split] for attn_decode_merge_kernel, which also forms the
+// O projection's input code (one launch, as the quantization alone).  385 queries after 3000 keys (50 query
+// tiles): 131 -> 39 us and the merge 7 us
+// where the quantization took 5; 512 queries: 24.5 -> 11 us.
 // ---------------------------------------------------------------------------------------------
 constexpr int kPfStages = 2;
 constexpr int kPfComputeWaves = QWEN_GROUPS;  // one per query head
 
-__global__ void __launch_bounds__(64 * (kPfComputeWaves + 1)) attn_prefill_tiles_kernel(const float* __restrict__ qkv, int qkv_stride,
-                                                                 const uint8_t* __restrict__ kvt, int S, int past,
-                                                                 float* __restrict__ ctx) {
+template <bool SPLIT>
+__global__ void __launch_bounds__(64 * (kPfComputeWaves + 1))
+attn_prefill_tiles_kernel(const float* __restrict__ qkv, int qkv_stride, const uint8_t* __restrict__ kvt, int S, int past,
+                          float* __restrict__ ctx, int nsplit, int tps, float* __restrict__ part,
+                          float2* __restrict__ pml) {
   __shared__ __align__(16) uint8_t stages[kPfStages][kPfTileBytes];
   const int nqt = gridDim.x;
   const int qt = nqt - 1 - blockIdx.x;  // longest rows first
   const int kvh = blockIdx.y;
-  const int sq = blockIdx.z;
+  const int sq = SPLIT ? blockIdx.z / nsplit : blockIdx.z;
+  const int split = SPLIT ? blockIdx.z % nsplit : 0;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int q0 = qt * kPfQ;                   // local query rows q0.. of the S new tokens
   const int nkeys = past + S;                 // keys of the sequence (past rows, then the new ones)
   const int qlast = past + min(q0 + kPfQ, S) - 1;  // last query position of the block
-  const int ntiles = qlast / kPfKeys + 1;     // key tiles 0 .. qlast/32 (causal)
+  const int tfirst = SPLIT ? split * tps : 0;
+  // key tiles tfirst .. of 0 .. qlast/32 (causal)
+  const int ntiles = SPLIT ? min(tps, qlast / kPfKeys + 1 - tfirst) : qlast / kPfKeys + 1;
+  if (SPLIT && ntiles <= 0) return;  // block-uniform: the queries' keys end before this split
   const int ntile_all = (nkeys + kPfKeys - 1) / kPfKeys;
-  const uint8_t* tiles = kvt + (size_t)(sq * 2 + kvh) * ntile_all * kPfTileBytes;
+  const uint8_t* tiles = kvt + ((size_t)(sq * 2 + kvh) * ntile_all + tfirst) * kPfTileBytes;
 
   if (wave >= kPfComputeWaves) {
     // producer: streams each 32 KiB tile, 32 loads of 1 KiB, one tile ahead
@@ -3614,12 +3631,13 @@ __global__ void __launch_bounds__(64 * (kPfComputeWaves + 1)) attn_prefill_tiles
       }
     }
     // Only a tile that reaches past the wave's first query or past the last key needs the mask.
-    if (t * kPfKeys + kPfKeys - 1 > qpos0 || t * kPfKeys + kPfKeys > nkeys) {
+    const int key0 = (tfirst + t) * kPfKeys;
+    if (key0 + kPfKeys - 1 > qpos0 || key0 + kPfKeys > nkeys) {
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int key = t * kPfKeys + kt * 16 + 4 * g + r;
+          const int key = key0 + kt * 16 + 4 * g + r;
           if (key > qpos || key >= nkeys) sc[kt][r] = -INFINITY;
         }
     }
@@ -3632,13 +3650,16 @@ __global__ void __launch_bounds__(64 * (kPfComputeWaves + 1)) attn_prefill_tiles
     // Tile 0 holds key 0 <= qpos, so m_run is finite from tile 0 on; a later tile with every key
     // past qpos gives mt = -inf, corr = 1 and p = 0, leaving the column's state unchanged.
     mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+    // A split may start past a query's last key: its column stays at -inf, and a zero reference keeps the
+    // exponentials at 0 (the merge does not read such a column).
     const float mn = fmaxf(m_run, mt);
-    const float corr = __expf(m_run - mn);
+    const float mref = SPLIT && mn == -INFINITY ? 0.0f : mn;
+    const float corr = __expf(m_run - mref);
     float p[8];
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) p[kt * 4 + r] = __expf(sc[kt][r] - mn);
+      for (int r = 0; r < 4; ++r) p[kt * 4 + r] = __expf(sc[kt][r] - mref);
     l_run = l_run * corr + (((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7])));
     m_run = mn;
     bf16x8 ph, pl;
@@ -3672,6 +3693,20 @@ __global__ void __launch_bounds__(64 * (kPfComputeWaves + 1)) attn_prefill_tiles
   float lp = l_run;
   lp += __shfl_xor(lp, 16, 64);
   lp += __shfl_xor(lp, 32, 64);
+  if (SPLIT) {
+    if (g == 0 && q0 + col < S)
+      pml[(((size_t)sq * S + q0 + col) * QWEN_Q_HEADS + h) * nsplit + split] = make_float2(m_run, lp);
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) {
+      const int qi = q0 + 4 * g + rr;
+      if (qi < S) {
+        float* op = part + ((((size_t)sq * S + qi) * QWEN_Q_HEADS + h) * nsplit + split) * QWEN_HEAD_DIM + col;
+#pragma unroll
+        for (int n = 0; n < 8; ++n) op[16 * n] = acc[n][rr];
+      }
+    }
+    return;
+  }
   const float inv = lp > 0.0f ? 1.0f / lp : 0.0f;  // of query column col
 #pragma unroll
   for (int rr = 0; rr < 4; ++rr) {
@@ -3848,8 +3883,31 @@ static int split_for(int nkc, int want) {
   return 1;
 }
 
-// Shape dispatch (the split-K workspace a.part, when given, holds kMaxSplits x kSplitTokens x
-// out_dim floats).  <= 16 tokens: direct-load kernel, 4-way in-block K split per row tile (many
+// K splits of the two-blocks-per-CU pipelined GEMM for more than kSplitTokens tokens: the least of the time
+// of its rounds (0.9 us per K chunk of a block alone on its CU, 1.64 us of two) and of the partials' write and
+// read, 2 us for the reduce launch where the call has none anyway.  512 tokens: the down projection's 48
+// blocks of 70 chunks 63.5 us, in 5 splits 21.5 us and its
+// reduce step 7.1 us (which carries the next RMSNorm + quantization, 5.2 us as a launch of its own).
+static int pipe_splits(const GemmArgs& a, int nkc, int row_tiles) {
+  if (!a.part || a.out_dim > QWEN_QKV_ROWS) return 1;
+  const int blocks = (a.tokens + 63) / 64 * ((row_tiles + 15) / 16);
+  int best = 1;
+  double cost = 0.0;
+  for (int s = 1; s <= kMaxSplits; ++s) {
+    if (nkc % s != 0 || s * a.tokens > kSplitRows) continue;
+    const int n = blocks * s;
+    const double rounds = n <= 256 ? 0.9 : 1.64 * ((n + 511) / 512);
+    const double c = rounds * (nkc / s) + (s > 1 || a.fuse != kFuseNone ? s * (double)a.tokens * a.out_dim * 8.0 / 4.5e6 : 0.0) +
+                     (s > 1 && a.fuse == kFuseNone ? 2.0 : 0.0);
+    if (s == 1 || c < cost) {
+      cost = c;
+      best = s;
+    }
+  }
+  return best;
+}
+
+// Shape dispatch (the split-K workspace a.part, when given, holds kSplitRows x out_dim floats).  <= 16 tokens: direct-load kernel, 4-way in-block K split per row tile (many
 // small blocks, weights streamed once).  More tokens: the pipelined LDS kernel; projections whose
 // row tiles alone give fewer than ~256 blocks are also split over K across blocks (needs a.part).
 template <int EPI, bool DUAL>
@@ -3877,24 +3935,28 @@ static void launch_gemm_epi(const GemmArgs& a, hipStream_t st) {
     if (!DUAL && a.fuse != kFuseNone) launch_reduce<EPI>(a, 1, st);
     return;
   }
+  if constexpr (!DUAL && EPI == kEpiStore) {
+    if (a.fuse == kFuseRopePrefill) {
+      if (a.tokens <= kSkinnyTokens || a.out_dim != QWEN_QKV_ROWS || a.seq_len <= 0 || a.past < 0 || !a.rope ||
+          !a.k_cache || !a.v_cache)
+        throw std::runtime_error("prefill RoPE epilogue: more than 64 tokens of the [q | k | v] projection");
+      // one head per block while two-head blocks (8 per 64 tokens) do not fill the CUs: 512 tokens 17.2 -> 12.0 us
+      if ((a.tokens + 63) / 64 * 8 <= 256)
+        launch_gemm_pipe_t<4, 2, 2, EPI, DUAL, 1, 2, true, true>(a, 1, st);
+      else
+        launch_gemm_pipe_t<4, 4, 2, EPI, DUAL, 1, 2, true, true>(a, 1, st);
+      return;
+    }
+  }
   // Many tokens (prefill): 4-wave blocks of 64 tokens with two LDS stages (64 KiB), two blocks per
   // CU.  Measured against one 8-wave block of 128 tokens with three stages (144 KiB) per CU at 16,384
   // tokens: gate/up 0.94-0.98 -> 0.79 ms, down 0.38-0.40 -> 0.34 ms, QKV 111-118 -> 97-100 us.
-  if (a.tokens > kSplitTokens && a.fuse == kFuseNone) {
+  if (a.tokens > kSplitTokens) {
     if constexpr (DUAL)
       launch_gemm_pipe_t<4, 2, 2, EPI, DUAL, 1, 2, true>(a, 1, st);
     else
-      launch_gemm_pipe_t<4, 4, 2, EPI, DUAL, 1, 2, true>(a, 1, st);
+      launch_gemm_pipe_t<4, 4, 2, EPI, DUAL, 1, 2, true>(a, pipe_splits(a, nkc, row_tiles), st);
     return;
-  }
-  if constexpr (!DUAL && EPI == kEpiStore) {
-    if (a.fuse == kFuseRopePrefill) {
-      if (a.tokens <= kSplitTokens || a.out_dim != QWEN_QKV_ROWS || a.seq_len <= 0 || a.past < 0 || !a.rope ||
-          !a.k_cache || !a.v_cache)
-        throw std::runtime_error("prefill RoPE epilogue: more than 256 tokens of the [q | k | v] projection");
-      launch_gemm_pipe_t<4, 4, 2, EPI, DUAL, 1, 2, true, true>(a, 1, st);
-      return;
-    }
   }
   if constexpr (DUAL) {
     if (a.tokens <= 64)
@@ -4104,24 +4166,62 @@ void launch_attn_decode(const float* qkv, int qkv_stride, const float* k_cache, 
   hipLaunchKernelGGL(attn_decode_kernel, dim3(plan.nsplit, QWEN_KV_HEADS, batch), dim3(256), 0, st, qkv, qkv_stride,
                      k_cache, v_cache, seq_stride, pos, plan.chunk, max_keys, part, pml);
   if (xq)
-    hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(batch), dim3(256), 0, st, part, pml, pos, plan.nsplit, plan.chunk,
-                       max_keys, ctx, xq, sx, sums);
+    hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(batch), dim3(256), 0, st, part, pml, pos, 1, 0, plan.nsplit,
+                       plan.chunk, max_keys, ctx, xq, sx, sums);
 }
 
 size_t attn_prefill_workspace_bytes(int keys, int nseq) {
   return (size_t)nseq * QWEN_KV_HEADS * ((keys + kPfKeys - 1) / kPfKeys) * kPfTileBytes;
 }
 
+AttnPrefillPlan plan_attn_prefill(int S, int past, int nseq) {
+  const int ntiles = (past + S + kPfKeys - 1) / kPfKeys;
+  const int qtiles = (S + kPfQ - 1) / kPfQ;
+  AttnPrefillPlan best{1, ntiles};
+  double cost = 0.0;
+  // The time in tiles of a block alone on its CU (1.2 us): its tiles and about 4 for its start and end while
+  // every block has a CU; two blocks on a CU take 2.2 times as long per tile, and the CUs share what there
+  // is.  The partials' write and read add 100 KB per block.
+  for (int n = 1; n <= kAttnMaxSplits && n <= ntiles; ++n) {
+    const int tps = (ntiles + n - 1) / n;
+    if (n > 1 && tps == (ntiles + n - 2) / (n - 1)) continue;  // same tiles per split: fewer splits
+    double total = 0.0, blocks = 0.0;
+    for (int q = 0; q < qtiles; ++q) {
+      const int last = past + (q * kPfQ + kPfQ < S ? q * kPfQ + kPfQ : S) - 1;
+      total += last / kPfKeys + 1;
+      blocks += last / kPfKeys / tps + 1;
+    }
+    total *= 2.0 * nseq;
+    blocks *= 2.0 * nseq;
+    const double alone = tps + 4.0, share = 1.1 * (total + 4.0 * blocks) / 256.0;
+    const double c = (blocks <= 256.0 ? alone : share > 2.2 * alone ? share : 2.2 * alone) + (n > 1 ? blocks * 0.03 : 0.0);
+    if (n == 1 || c < cost) {
+      cost = c;
+      best = AttnPrefillPlan{n, tps};
+    }
+  }
+  return best;
+}
+
 void launch_attn_prefill(const float* qkv, int qkv_stride, const float* k_cache, const float* v_cache,
-                         size_t seq_stride, int S, int past, int nseq, uint8_t* kv_tiles, float* ctx,
-                         hipStream_t st) {
+                         size_t seq_stride, int S, int past, int nseq, uint8_t* kv_tiles, const AttnPrefillPlan& plan,
+                         float* part, float2* pml, float* ctx, int8_t* xq, float* sx, int* sums, hipStream_t st) {
   const int keys = past + S;
   const int ntile = (keys + kPfKeys - 1) / kPfKeys;
   hipLaunchKernelGGL(kv_bf16_tiles_kernel, dim3(ntile, QWEN_KV_HEADS, nseq), dim3(256), 0, st, k_cache, v_cache,
                      seq_stride, keys, kv_tiles);
-  hipLaunchKernelGGL(attn_prefill_tiles_kernel, dim3((S + kPfQ - 1) / kPfQ, QWEN_KV_HEADS, nseq),
-                     dim3(64 * (kPfComputeWaves + 1)), 0, st,
-                     qkv, qkv_stride, kv_tiles, S, past, ctx);
+  const dim3 grid((S + kPfQ - 1) / kPfQ, QWEN_KV_HEADS, nseq * plan.nsplit);
+  const dim3 block(64 * (kPfComputeWaves + 1));
+  if (plan.nsplit > 1) {
+    hipLaunchKernelGGL(attn_prefill_tiles_kernel<true>, grid, block, 0, st, qkv, qkv_stride, kv_tiles, S, past, ctx,
+                       plan.nsplit, plan.tps, part, pml);
+    hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(nseq * S), dim3(256), 0, st, part, pml,
+                       static_cast<const int*>(nullptr), S, past, plan.nsplit, plan.tps * kPfKeys, keys,
+                       static_cast<float*>(nullptr), xq, sx, sums);
+    return;
+  }
+  hipLaunchKernelGGL(attn_prefill_tiles_kernel<false>, grid, block, 0, st, qkv, qkv_stride, kv_tiles, S, past, ctx, 1, 0,
+                     part, pml);
 }
 
 void launch_round_bf16(float* x, size_t n, hipStream_t st) {

@@ -139,6 +139,10 @@ struct qwen_hip_model {
               reinterpret_cast<const int*>(b + o_zs), reinterpret_cast<float*>(b + o_gmax)};
   }
 
+  Ws carve_prefill(size_t tokens, int nseq, int keys, const AttnPrefillPlan& plan) {
+    return carve(tokens, plan.nsplit > 1 ? tokens : 1, plan.nsplit, attn_prefill_workspace_bytes(keys, nseq));
+  }
+
   // Plain scratch of `bytes` in the workspace, past the fixed region.
   float* scratch(size_t bytes) {
     const size_t off = kFixedBytes;
@@ -433,14 +437,25 @@ struct qwen_hip_model {
   void prefill_fast(int first, int count, int B, int S, int past, float* hidden, float* kc0, float* vc0, uint64_t ss,
                     uint64_t ls, int round) {
     const int T = B * S;
-    const Ws w = carve(T, 1, 1, attn_prefill_workspace_bytes(past + S, B));
+    const AttnPrefillPlan plan = plan_attn_prefill(S, past, B);
+    const Ws w = carve_prefill(T, B, past + S, plan);
+    // Up to kPrefillFuseTokens tokens the RMSNorm + quantization that follow the O and down projections run in
+    // the step that adds those projections' K splits (their 64-token tiles alone fill a fraction of the CUs).
+    const bool fused = T > kSkinnyTokens && T <= kPrefillFuseTokens;
+    GemmArgs fn{};
+    fn.fuse = kFuseNormQuant;
+    fn.norm = kNormPrefill;
+    fn.xq_out = w.xq;
+    fn.sx_out = w.sx;
+    fn.sums_out = w.sums;
     for (int i = 0; i < count; ++i) {
       const FastLayer& f = fast[first + i];
       float* kc = kc0 + (size_t)i * ls;
       float* vc = vc0 + (size_t)i * ls;
-      launch_norm_quant(hidden, QWEN_HIDDEN, T, QWEN_HIDDEN, f.ln, kNormPrefill, w.xq, w.sx, w.sums, nullptr,
-                        stream);
-      if (T > kSplitTokens) {
+      if (!fused || i == 0)
+        launch_norm_quant(hidden, QWEN_HIDDEN, T, QWEN_HIDDEN, f.ln, kNormPrefill, w.xq, w.sx, w.sums, nullptr,
+                          stream);
+      if (T > kSkinnyTokens) {
         // RoPE of q and k and the K/V cache append in the Q/K/V projection's epilogue
         GemmArgs fr{};
         fr.fuse = kFuseRopePrefill;
@@ -457,17 +472,24 @@ struct qwen_hip_model {
         gemm(w, T, QWEN_HIDDEN, (int)kQkvRows, f.qkv, f.sw_qkv, f.b_qkv, w.qkv, kQkvRows, kEpiStore);
         launch_rope_qkv(w.qkv, (int)kQkvRows, nullptr, S, past, past + S, T, rope_prefill, kc, vc, ss, stream);
       }
-      launch_attn_prefill(w.qkv, (int)kQkvRows, kc, vc, ss, S, past, B, w.kvt, w.ctx, stream);
-      launch_norm_quant(w.ctx, QWEN_HIDDEN, T, QWEN_HIDDEN, nullptr, kNormNone, w.xq, w.sx, w.sums, nullptr, stream);
-      gemm(w, T, QWEN_HIDDEN, QWEN_HIDDEN, f.o, f.sw_o, nullptr, w.att, QWEN_HIDDEN, kEpiStore);
-      launch_norm_quant(w.att, QWEN_HIDDEN, T, QWEN_HIDDEN, f.post_ln, kNormPrefill, w.xq, w.sx, w.sums, nullptr,
-                        stream);
+      launch_attn_prefill(w.qkv, (int)kQkvRows, kc, vc, ss, S, past, B, w.kvt, plan, w.part, w.pml, w.ctx, w.xq, w.sx,
+                          w.sums, stream);
+      if (plan.nsplit == 1)
+        launch_norm_quant(w.ctx, QWEN_HIDDEN, T, QWEN_HIDDEN, nullptr, kNormNone, w.xq, w.sx, w.sums, nullptr, stream);
+      fn.norm_w = f.post_ln;
+      gemm(w, T, QWEN_HIDDEN, QWEN_HIDDEN, f.o, f.sw_o, nullptr, w.att, QWEN_HIDDEN, kEpiStore, nullptr, nullptr,
+           nullptr, 0, 0, fused ? &fn : nullptr);
+      if (!fused)
+        launch_norm_quant(w.att, QWEN_HIDDEN, T, QWEN_HIDDEN, f.post_ln, kNormPrefill, w.xq, w.sx, w.sums, nullptr,
+                          stream);
       gemm(w, T, QWEN_HIDDEN, QWEN_INTERMEDIATE, f.gate, f.sw_gate, nullptr, w.s, QWEN_INTERMEDIATE, kEpiSiluMul,
            f.up, f.sw_up, nullptr, 0, 1);
       launch_norm_quant(w.s, QWEN_INTERMEDIATE, T, QWEN_INTERMEDIATE, nullptr, kNormNone, w.xq, w.sx, w.sums,
                         nullptr, stream);
+      const bool fuse_next = fused && i + 1 < count;  // the next layer's input RMSNorm + quantize
+      fn.norm_w = fuse_next ? fast[first + i + 1].ln : nullptr;
       gemm(w, T, QWEN_INTERMEDIATE, QWEN_HIDDEN, f.down, f.sw_down, nullptr, hidden, QWEN_HIDDEN, kEpiResidual,
-           nullptr, nullptr, w.att, round, 0);
+           nullptr, nullptr, w.att, round, 0, fuse_next ? &fn : nullptr);
     }
     QWEN_HIP(hipGetLastError());
   }
@@ -803,8 +825,9 @@ int qwen_hip_model_time_kernel(qwen_hip_model* m, int kernel, int layer, int rep
   return guarded_model([&]() -> int {
     const int T = c.batch * c.seq_len;
     const AttnDecodePlan plan = plan_attn_decode(decode ? c.batch : 1, c.max_keys);
-    const qwen_hip_model::Ws w = m->carve(T, decode ? c.batch : 1, decode ? plan.nsplit : 1,
-                                          decode ? 0 : attn_prefill_workspace_bytes(c.max_keys, c.batch));
+    const AttnPrefillPlan pplan = decode ? AttnPrefillPlan{1, 1} : plan_attn_prefill(c.seq_len, c.past, c.batch);
+    const qwen_hip_model::Ws w =
+        decode ? m->carve(T, c.batch, plan.nsplit) : m->carve_prefill(T, c.batch, c.max_keys, pplan);
     const FastLayer& f = m->fast[layer];
     float* kc = c.k_cache + (size_t)(layer - c.first) * c.layer_stride;
     float* vc = c.v_cache + (size_t)(layer - c.first) * c.layer_stride;
@@ -835,8 +858,8 @@ int qwen_hip_model_time_kernel(qwen_hip_model* m, int kernel, int layer, int rep
           m->gemm(w, T, QWEN_HIDDEN, QWEN_HIDDEN, f.o, f.sw_o, nullptr, w.tmp, QWEN_HIDDEN, kEpiStore);
           break;
         case QWEN_KERNEL_ATTN_PREFILL:
-          launch_attn_prefill(w.qkv, (int)kQkvRows, kc, vc, c.seq_stride, c.seq_len, c.past, c.batch, w.kvt, w.ctx,
-                              m->stream);
+          launch_attn_prefill(w.qkv, (int)kQkvRows, kc, vc, c.seq_stride, c.seq_len, c.past, c.batch, w.kvt, pplan,
+                              w.part, w.pml, w.ctx, w.xq, w.sx, w.sums, m->stream);
           break;
         default:
           throw std::runtime_error("unknown kernel id");
