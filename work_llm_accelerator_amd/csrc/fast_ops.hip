@@ -73,7 +73,7 @@ int qwen_hip_fast_project(const uint8_t* w, const float* sw, const float* bias, 
     ScopedDev xq(xq_bytes((size_t)tokens, (size_t)in_dim));
     ScopedDev sx((size_t)tokens * 4u);
     ScopedDev sums((size_t)tokens * 8u);
-    ScopedDev part(splitk ? splitk_bytes((size_t)out_dim) : 256u);
+    ScopedDev part(splitk ? splitk_bytes((size_t)out_dim, (size_t)tokens) : 256u);
     launch_repack_int4(w, out_dim, in_dim, wp.as<uint8_t>(), st);
     launch_norm_quant(x, (size_t)in_dim, tokens, in_dim, nullptr, kNormNone, xq.as<int8_t>(), sx.as<float>(),
                       sums.as<int>(), nullptr, st);
@@ -149,7 +149,7 @@ int qwen_hip_fast_project_grouped(const uint8_t* w, const float* sw, int out_dim
     const int in = QWEN_INTERMEDIATE;
     ScopedDev wp((size_t)out_dim * in / 2);
     ScopedDev zero((size_t)tokens * 8u);  // limb sums of a code whose offsets are applied per group
-    ScopedDev part(splitk_bytes((size_t)out_dim));
+    ScopedDev part(splitk_bytes((size_t)out_dim, (size_t)tokens));
     launch_repack_int4(w, out_dim, in, wp.as<uint8_t>(), st);
     launch_zero_u32(zero.as<unsigned>(), 2 * tokens, st);
     GemmArgs a{};

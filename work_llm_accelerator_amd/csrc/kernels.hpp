@@ -160,7 +160,7 @@ struct GemmArgs {
 };
 
 // K splits across blocks: at most kMaxSplits splits and kSplitRows rows (splits x tokens) of partials;
-// the workspace holds kSplitRows x out floats.  kSplitTokens: the largest decode batch whose reduce steps
+// the workspace holds min(kMaxSplits x tokens, kSplitRows) x out floats.  kSplitTokens: the largest decode batch whose reduce steps
 // carry the fused epilogues; kPrefillFuseTokens: the same for the RMSNorm + quantization of a prefill.
 constexpr int kMaxSplits = 16;
 constexpr int kSplitTokens = 256;
@@ -175,7 +175,9 @@ constexpr int kPreResidualSplits = 5;
 constexpr int kOneTokenOSplits = 2;
 // Decode GEMMs of at most kSkinnyTokens tokens (in_dim 1536 or 8960) run the skinny kernels.
 constexpr int kSkinnyTokens = 64;
-inline size_t splitk_bytes(size_t out) { return (size_t)kSplitRows * out * 4u; }
+inline size_t splitk_bytes(size_t out, size_t tokens) {
+  return (tokens < kSplitRows / kMaxSplits ? kMaxSplits * tokens : (size_t)kSplitRows) * out * 4u;
+}
 
 void launch_repack_int4(const uint8_t* W, int out_dim, int in_dim, uint8_t* WP, hipStream_t st);
 void launch_norm_quant(const float* x, size_t x_stride, int rows, int n, const float* w, int norm, int8_t* xq,
@@ -220,15 +222,19 @@ void launch_rope_qkv(float* qkv, int qkv_stride, const int* pos, int seq_len, in
 // floats, pml [batch][12][nsplit] (m, l) pairs.  launch_attn_decode leaves the split partials there,
 // then (xq given) merges them into the context row, written to ctx when given, and its two-limb
 // code (xq, sx, sums); batch <= 65535 (one grid z index per sequence).
+// ragged_blocks > 0 (more than 64 sequences): the blocks per KV head over which the launch divides the
+// batch's own key counts on the device (at most nsplit splits of a sequence; budget: one int of workspace
+// that carries the key budget of a block to the merge).
 struct AttnDecodePlan {
-  int nsplit, chunk;
+  int nsplit, chunk, ragged_blocks;
 };
 // `cus`: the CUs the launch may use (a CU-masked stream), 0 for all of them.
 AttnDecodePlan plan_attn_decode(int batch, int max_keys, int cus = 0);
 void launch_zero_u32(unsigned* p, int n, hipStream_t st);
 void launch_attn_decode(const float* qkv, int qkv_stride, const float* k_cache, const float* v_cache,
                         size_t seq_stride, const int* pos, int batch, int max_keys, const AttnDecodePlan& plan,
-                        float* part, float2* pml, float* ctx, int8_t* xq, float* sx, int* sums, hipStream_t st);
+                        float* part, float2* pml, int* budget, float* ctx, int8_t* xq, float* sx, int* sums,
+                        hipStream_t st);
 // Prefill attention of S new tokens per sequence at positions past..past+S-1 over the cache rows
 // 0..past+S-1: K/V converted once into bf16 hi/lo tiles (workspace of
 // attn_prefill_workspace_bytes(past + S, nseq)), then the causal attention over them into ctx.  The plan

@@ -708,7 +708,9 @@ constexpr int kIntSumMaxK = 8192;
 // its accumulator slot 0, and the wave runs half of that slot's MFMAs before the chunk's barrier (its
 // own loads have landed by its own wait), so waves that reach the barrier late are absorbed by matrix
 // work instead of stalling the others.  Slot n holds token tile (wv + n) mod 4.
-// ROPE (the fused [q | k | v] projection of a prefill, kFuseRopePrefill): wave w of a block (RTW = 4: 2 heads,
+// ROPE (the fused [q | k | v] projection of a prefill, kFuseRopePrefill, or of a decode batch, kFuseQkvRope:
+// token t at position pos[t] of sequence t, a position outside [0, limit) leaving q unrotated and the cache
+// untouched): wave w of a block (RTW = 4: 2 heads,
 // 16 row tiles) holds row tiles h*8 + 2*(w & 1) + {0, 1} and the same + 4 of head h = w >> 1, so that
 // tiles r and r + 2 hold the rotation pairs (p, p + 64) of one head and the epilogue rotates q and k and
 // appends K/V to the cache, as rope_qkv_kernel does after a plain store.  RTW = 2 (one head per block, for
@@ -938,15 +940,16 @@ __global__ void __launch_bounds__(256 * TW) __attribute__((amdgpu_waves_per_eu(W
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
           const int tc = min(tok[n], a.tokens - 1);
-          seqn[n] = tc / a.seq_len;
-          Pn[n] = a.past + tc % a.seq_len;
+          seqn[n] = a.pos ? tc : tc / a.seq_len;
+          Pn[n] = a.pos ? a.pos[tc] : a.past + tc % a.seq_len;
           const int Pc = min(max(Pn[n], 0), a.limit - 1);
           cs[n] = *reinterpret_cast<const float4*>(a.rope + (size_t)Pc * 128 + p);
           sn[n] = *reinterpret_cast<const float4*>(a.rope + (size_t)Pc * 128 + 64 + p);
         }
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
-          if (tok[n] >= a.tokens || Pn[n] < 0 || Pn[n] >= a.limit) continue;
+          const bool in = Pn[n] >= 0 && Pn[n] < a.limit;
+          if (tok[n] >= a.tokens || (!in && head >= QWEN_Q_HEADS)) continue;
           float e[4], od[4];
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
@@ -959,9 +962,9 @@ __global__ void __launch_bounds__(256 * TW) __attribute__((amdgpu_waves_per_eu(W
           float lo[4], hi[4];
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            const bool v_head = head >= QWEN_Q_HEADS + QWEN_KV_HEADS;
-            lo[q] = v_head ? e[q] : e[q] * c4[q] - od[q] * s4[q];
-            hi[q] = v_head ? od[q] : od[q] * c4[q] + e[q] * s4[q];
+            const bool plain = head >= QWEN_Q_HEADS + QWEN_KV_HEADS || !in;
+            lo[q] = plain ? e[q] : e[q] * c4[q] - od[q] * s4[q];
+            hi[q] = plain ? od[q] : od[q] * c4[q] + e[q] * s4[q];
           }
           float* dst;
           if (head < QWEN_Q_HEADS) {
@@ -2577,80 +2580,6 @@ __global__ void __launch_bounds__(256) gemm_splitk_reduce_kernel(GemmArgs a, int
   *reinterpret_cast<float4*>(a.y + (size_t)tok * a.y_stride + row0) = make_float4(out[0], out[1], out[2], out[3]);
 }
 
-// Finishes output (tok, row) from its split sum: offset correction and bias, the same arithmetic as
-// gemm_splitk_reduce_kernel.
-__device__ __forceinline__ float finish_one(const GemmArgs& a, float acc, int row, double corr) {
-  return acc + (float)(corr * (double)a.sw[row]) + (a.bias ? a.bias[row] : 0.0f);
-}
-
-// kFuseQkvRope: reduce of the fused [q | k | v] projection (2048 rows) for decode token t, bias, RoPE
-// of the 12 q heads (in place in a.y) and the 2 k heads, and the K/V cache append at position
-// pos[t] of sequence t (qwen_decode_attention_kernel.cpp:29-42,100-111 semantics; positions outside
-// [0, limit) leave q unrotated and the cache untouched).  Thread t of the block owns rotation pair
-// p = t & 63 of heads (t >> 6) + 4k, k < 4 (heads 0-11 q, 12-13 k, 14-15 v).  grid = tokens, block = 256.
-__global__ void __launch_bounds__(256) reduce_qkv_rope_kernel(GemmArgs a, int splits) {
-  const int tok = blockIdx.x;
-  const int p = threadIdx.x & 63;
-  const double corr = -8.0 * (256.0 * (double)a.sums[2 * tok] + (double)a.sums[2 * tok + 1]) * (double)a.sx[tok];
-  const int P = a.pos[tok];
-  const bool in = P >= 0 && P < a.limit;
-  float c = 1.0f, sn = 0.0f;
-  if (in) {
-    c = a.rope[(size_t)P * 128 + p];
-    sn = a.rope[(size_t)P * 128 + 64 + p];
-  }
-  float* yq = a.y + (size_t)tok * a.y_stride;
-  float* kc = a.k_cache + (size_t)tok * a.seq_stride + (size_t)(in ? P : 0) * QWEN_KV_WIDTH;
-  float* vc = a.v_cache + (size_t)tok * a.seq_stride + (size_t)(in ? P : 0) * QWEN_KV_WIDTH;
-  // split sums of the thread's 8 rows (4 pairs), 4 splits per batch of loads, in z order
-  const size_t zstride = (size_t)a.tokens * a.out_dim;
-  const float* pt = a.part + (size_t)tok * a.out_dim + p;
-  float sum[4][2];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) sum[k][0] = sum[k][1] = 0.0f;
-  for (int z0 = 0; z0 < splits; z0 += 4) {
-    float pz[4][4][2];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-#pragma unroll
-        for (int hh = 0; hh < 2; ++hh)
-          pz[u][k][hh] = z0 + u < splits
-                             ? pt[(size_t)(z0 + u) * zstride + ((threadIdx.x >> 6) + 4 * k) * QWEN_HEAD_DIM + 64 * hh]
-                             : 0.0f;
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (z0 + u < splits)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          sum[k][0] += pz[u][k][0];
-          sum[k][1] += pz[u][k][1];
-        }
-  }
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int head = (threadIdx.x >> 6) + 4 * k;
-    const int r0 = head * QWEN_HEAD_DIM + p;
-    const float e = finish_one(a, sum[k][0], r0, corr);
-    const float od = finish_one(a, sum[k][1], r0 + 64, corr);
-    if (head < QWEN_Q_HEADS) {
-      yq[r0] = in ? e * c - od * sn : e;
-      yq[r0 + 64] = in ? od * c + e * sn : od;
-    } else if (!in) {
-      continue;
-    } else if (head < QWEN_Q_HEADS + QWEN_KV_HEADS) {
-      const int base = (head - QWEN_Q_HEADS) * QWEN_HEAD_DIM + p;
-      kc[base] = e * c - od * sn;
-      kc[base + 64] = od * c + e * sn;
-    } else {
-      const int base = (head - QWEN_Q_HEADS - QWEN_KV_HEADS) * QWEN_HEAD_DIM + p;
-      vc[base] = e;
-      vc[base + 64] = od;
-    }
-  }
-}
-
 // kFuseNormQuant: reduce of a 1536-row projection for token t with the EPI epilogue (kEpiStore: bias;
 // kEpiResidual: residual, optional raw copy, optional bf16 rounding), the finished row written to
 // a.y, then RMSNorm(norm_w) + two-limb quantization of that row into xq_out / sx_out / sums_out.
@@ -3229,10 +3158,31 @@ __device__ __forceinline__ void attn_decode_tile(const float* __restrict__ kb, c
   attn_decode_tile_math<MASK>(qrow, tb, t1, g, m, lp, acc, kr, vr);
 }
 
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
-attn_decode_kernel(const float* __restrict__ qkv, int qkv_stride, const float* __restrict__ k_cache,
-                   const float* __restrict__ v_cache, size_t seq_stride, const int* __restrict__ pos, int chunk,
-                   int max_keys, float* __restrict__ part, float2* __restrict__ pml) {
+constexpr int kAttnMinChunk = 64;
+
+// Ragged batches (RAGGED; more than kRaggedFrom sequences, where the device holds only two or three splits of
+// each sequence at once): one chunk size from the longest sequence leaves the blocks of short ones nearly
+// empty.  Every block instead derives the split from the batch's own lengths n_s: a key budget per block
+//   C = max(kAttnMinChunk, longest / max_splits, sum n_s / (blocks - batch / 2)) in whole 16-key tiles,
+//   k_s = ceil(n_s / C) splits of chunk_s = ceil(n_s / k_s) keys,
+// and finds its own (sequence, KV head, split) by a prefix sum over k_s, in the same order as the plain grid.
+// C goes to *budget for the merge.  150 sequences of 100 to 900 keys: 51 us with one
+// chunk size, 34 us so (154 MB of K/V rows); of 900 keys each the whole layer step is 5 us shorter too.
+struct RaggedArgs {
+  int batch, blocks, max_splits;  // blocks: per KV head
+  int* budget;
+};
+__device__ __forceinline__ int ragged_chunk(int n, int budget) {
+  const int k = (n + budget - 1) / budget;
+  return ((n + k - 1) / k + 15) & ~15;
+}
+
+template <bool RAGGED>
+__device__ __forceinline__ void attn_decode_body(const float* __restrict__ qkv, int qkv_stride,
+                                                 const float* __restrict__ k_cache, const float* __restrict__ v_cache,
+                                                 size_t seq_stride, const int* __restrict__ pos, int chunk, int max_keys,
+                                                 float* __restrict__ part, float2* __restrict__ pml,
+                                                 const RaggedArgs& ra) {
   // (the leading 14 argument dwords, through max_keys, are preloaded: the first loads wait for nothing;
   // the segment's other lines are requested at entry and waited for once the first tile is in flight)
   const auto klines = kernarg_lines_issue<
@@ -3240,14 +3190,70 @@ attn_decode_kernel(const float* __restrict__ qkv, int qkv_stride, const float* _
   __shared__ __align__(16) float qs[16][kQRow];
   __shared__ __align__(16) float s_acc[4][QWEN_GROUPS][QWEN_HEAD_DIM];
   __shared__ float s_m[4][QWEN_GROUPS], s_l[4][QWEN_GROUPS];
-  const int nsplit = gridDim.x;
-  const int c = blockIdx.x;
-  const int kvh = blockIdx.y;
-  const int b = blockIdx.z;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int col = lane & 15;
   const int g = lane >> 4;
+  int nsplit = gridDim.x, c = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
+  if constexpr (RAGGED) {
+    __shared__ int scan[2][4];
+    __shared__ int mine[4];
+    nsplit = ra.max_splits;
+    // thread t owns sequences t * per .. of the batch
+    const int per = (ra.batch + 255) / 256, s0 = threadIdx.x * per, s1 = min(s0 + per, ra.batch);
+    int total = 0, longest = 0;
+    for (int s = s0; s < s1; ++s) {
+      const int n = min(max(pos[s], 0) + 1, max_keys);
+      total += n;
+      longest = max(longest, n);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      total += __shfl_xor(total, off, 64);
+      longest = max(longest, __shfl_xor(longest, off, 64));
+    }
+    if (lane == 0) {
+      scan[0][wave] = total;
+      scan[1][wave] = longest;
+    }
+    if (threadIdx.x == 0) mine[0] = -1;
+    __syncthreads();
+    total = scan[0][0] + scan[0][1] + scan[0][2] + scan[0][3];
+    longest = max(max(scan[1][0], scan[1][1]), max(scan[1][2], scan[1][3]));
+    const int share = ra.blocks - ra.batch / 2;  // (the launcher keeps it positive)
+    int budget = max(max(kAttnMinChunk, (longest + nsplit - 1) / nsplit), (total + share - 1) / share);
+    budget = (budget + 15) & ~15;
+    int own = 0;  // splits of this thread's sequences
+    for (int s = s0; s < s1; ++s) own += (min(max(pos[s], 0) + 1, max_keys) + budget - 1) / budget;
+    int before = own;  // inclusive prefix over the wave, then over the waves
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int o = __shfl_up(before, off, 64);
+      if (lane >= off) before += o;
+    }
+    __syncthreads();  // scan is read above
+    if (lane == 63) scan[0][wave] = before;
+    __syncthreads();
+    before -= own;
+    for (int w = 0; w < wave; ++w) before += scan[0][w];
+    for (int s = s0; s < s1; ++s) {  // both KV heads of a sequence: 2 k_s blocks
+      const int k = (min(max(pos[s], 0) + 1, max_keys) + budget - 1) / budget;
+      const int i = (int)blockIdx.x - 2 * before;
+      if (i >= 0 && i < 2 * k) {
+        mine[0] = s;
+        mine[1] = i / k;
+        mine[2] = i % k;
+      }
+      before += k;
+    }
+    __syncthreads();
+    b = mine[0];
+    if (blockIdx.x == 0 && threadIdx.x == 0) *ra.budget = budget;
+    if (b < 0) return;  // block-uniform: past the last sequence's blocks
+    kvh = mine[1];
+    c = mine[2];
+    chunk = ragged_chunk(min(max(pos[b], 0) + 1, max_keys), budget);
+  }
   const int n = min(max(pos[b], 0) + 1, max_keys);
   const int t0 = c * chunk;
   const float scaling = 0.08838834764831845f;
@@ -3349,28 +3355,43 @@ attn_decode_kernel(const float* __restrict__ qkv, int qkv_stride, const float* _
   }
 }
 
-// The split merge of attn_decode_kernel's partials, one block per sequence (pos given), or of the split prefill
-// attention's, one block per token (pos null: token b at position past + b % seq_len): per head the merge
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+attn_decode_kernel(const float* __restrict__ qkv, int qkv_stride, const float* __restrict__ k_cache,
+                   const float* __restrict__ v_cache, size_t seq_stride, const int* __restrict__ pos, int chunk,
+                   int max_keys, float* __restrict__ part, float2* __restrict__ pml) {
+  attn_decode_body<false>(qkv, qkv_stride, k_cache, v_cache, seq_stride, pos, chunk, max_keys, part, pml, RaggedArgs{});
+}
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+attn_decode_ragged_kernel(const float* __restrict__ qkv, int qkv_stride, const float* __restrict__ k_cache,
+                          const float* __restrict__ v_cache, size_t seq_stride, const int* __restrict__ pos,
+                          int max_keys, float* __restrict__ part, float2* __restrict__ pml, RaggedArgs ra) {
+  attn_decode_body<true>(qkv, qkv_stride, k_cache, v_cache, seq_stride, pos, 0, max_keys, part, pml, ra);
+}
+
+// The split merge of attn_decode_kernel's partials, one block per sequence (RAGGED: the splits follow from
+// *budget), or of the split prefill attention's, one block per token (token b at position past + b % seq_len):
+// per head the merge
 // weights of the splits that hold keys (merge_split_weights), the weighted sum of their partial rows
 // in split order into the context row (written to ctx when given), then the row's two-limb code,
 // scale and limb sums for the O projection (quantize_row_lds).  Thread t owns float4 columns t and
 // t + 256 (< 384) of the row.  Every load of a batch of 8 splits is issued unconditionally (splits
 // past the last one load the last again, unused) together with the (m, l) pairs, so sequences with
 // at most 8 splits need one memory round trip.
-__global__ void __launch_bounds__(256) attn_decode_merge_kernel(const float* __restrict__ part,
-                                                                const float2* __restrict__ pml,
-                                                                const int* __restrict__ pos, int seq_len, int past,
-                                                                int nsplit, int chunk, int max_keys,
-                                                                float* __restrict__ ctx,
-                                                                int8_t* __restrict__ xq, float* __restrict__ sx,
-                                                                int* __restrict__ sums) {
+constexpr int kMergeDecode = 0, kMergeRagged = 1, kMergePrefill = 2;
+template <int MODE>
+__device__ __forceinline__ void attn_merge_body(const float* __restrict__ part, const float2* __restrict__ pml,
+                                                const int* __restrict__ pos, int nsplit, int chunk, int max_keys,
+                                                float* __restrict__ ctx, int8_t* __restrict__ xq, float* __restrict__ sx,
+                                                int* __restrict__ sums, int seq_len, int past,
+                                                const int* __restrict__ budget) {
   constexpr int kF4 = QWEN_HIDDEN / 4;  // float4 columns of the row
   __shared__ __align__(16) float row[QWEN_HIDDEN];         // the context row
   __shared__ float ml[QWEN_Q_HEADS * kAttnMaxSplits * 2];  // (m, l), then merge weights in place
   __shared__ float red_f[4];
   __shared__ int red_i[8];
   const int b = blockIdx.x;
-  const int n = pos ? min(max(pos[b], 0) + 1, max_keys) : past + b % seq_len + 1;
+  const int n = MODE == kMergePrefill ? past + b % seq_len + 1 : min(max(pos[b], 0) + 1, max_keys);
+  if (MODE == kMergeRagged) chunk = ragged_chunk(n, *budget);
   const int nc = (n + chunk - 1) / chunk;  // splits that hold keys
   const float2* pb = pml + (size_t)b * QWEN_Q_HEADS * nsplit;
   const float* pa = part + (size_t)b * QWEN_Q_HEADS * nsplit * QWEN_HEAD_DIM;
@@ -3421,6 +3442,29 @@ __global__ void __launch_bounds__(256) attn_decode_merge_kernel(const float* __r
   }
   __syncthreads();
   quantize_row_lds(row, QWEN_HIDDEN, xq + (size_t)b * (2 * QWEN_HIDDEN), sx + b, sums + 2 * b, red_f, red_i);
+}
+
+__global__ void __launch_bounds__(256) attn_decode_merge_kernel(const float* __restrict__ part,
+                                                                const float2* __restrict__ pml,
+                                                                const int* __restrict__ pos, int nsplit, int chunk,
+                                                                int max_keys, float* __restrict__ ctx,
+                                                                int8_t* __restrict__ xq, float* __restrict__ sx,
+                                                                int* __restrict__ sums) {
+  attn_merge_body<kMergeDecode>(part, pml, pos, nsplit, chunk, max_keys, ctx, xq, sx, sums, 1, 0, nullptr);
+}
+__global__ void __launch_bounds__(256) attn_ragged_merge_kernel(const float* __restrict__ part,
+                                                                const float2* __restrict__ pml,
+                                                                const int* __restrict__ pos, int nsplit, int max_keys,
+                                                                const int* __restrict__ budget, float* __restrict__ ctx,
+                                                                int8_t* __restrict__ xq, float* __restrict__ sx,
+                                                                int* __restrict__ sums) {
+  attn_merge_body<kMergeRagged>(part, pml, pos, nsplit, 0, max_keys, ctx, xq, sx, sums, 1, 0, budget);
+}
+__global__ void __launch_bounds__(256) attn_prefill_merge_kernel(const float* __restrict__ part,
+                                                                 const float2* __restrict__ pml, int seq_len, int past,
+                                                                 int nsplit, int chunk, int8_t* __restrict__ xq,
+                                                                 float* __restrict__ sx, int* __restrict__ sums) {
+  attn_merge_body<kMergePrefill>(part, pml, nullptr, nsplit, chunk, 0, nullptr, xq, sx, sums, seq_len, past, nullptr);
 }
 
 __global__ void zero_u32_kernel(unsigned* __restrict__ p, int n) {
@@ -3532,7 +3576,7 @@ __global__ void __launch_bounds__(256) kv_bf16_tiles_kernel(const float* __restr
 // grid = (ceil(S/16), 2, nseq) with query tiles longest first, block = 448.
 // SPLIT: few query tiles leave most CUs idle, so the key tiles of a query tile go to several blocks of tps
 // tiles each (grid.z = nseq * nsplit); a block leaves its queries' unnormalized rows and (max, sum) in
-// part[token][head][split][128], pml[token][head][split] for attn_decode_merge_kernel, which also forms the
+// part[token][head][split][128], pml[token][head][split] for attn_prefill_merge_kernel, which also forms the
 // O projection's input code (one launch, as the quantization alone).  385 queries after 3000 keys (50 query
 // tiles): 131 -> 39 us and the merge 7 us
 // where the quantization took 5; 512 queries: 24.5 -> 11 us.
@@ -3764,9 +3808,7 @@ static void launch_gemm_t(const GemmArgs& a, hipStream_t st) {
 // The reduce step after a GEMM that wrote fp32 partials: plain (bias / residual epilogue) or fused.
 template <int EPI>
 static void launch_reduce(const GemmArgs& a, int splits, hipStream_t st) {
-  if (a.fuse == kFuseQkvRope) {
-    hipLaunchKernelGGL(reduce_qkv_rope_kernel, dim3(a.tokens), dim3(256), 0, st, a, splits);
-  } else if (a.fuse == kFuseNormQuant) {
+  if (a.fuse == kFuseNormQuant) {
     if (a.out_dim == QWEN_HIDDEN && splits <= 5 && (EPI != kEpiResidual || a.resid_stride == QWEN_HIDDEN)) {
       // the first loads' operands preloaded (an absent bias or norm weight read from the row scales)
       const void* add = EPI == kEpiResidual ? (const void*)a.resid : a.bias ? (const void*)a.bias : a.sw;
@@ -3876,27 +3918,19 @@ static bool launch_skinny(const GemmArgs& a, hipStream_t st) {
   return false;
 }
 
-// Largest divisor of nkc that is <= want (K chunks split evenly over blocks).
-static int split_for(int nkc, int want) {
-  for (int s = want < kMaxSplits ? want : kMaxSplits; s > 1; --s)
-    if (nkc % s == 0) return s;
-  return 1;
-}
-
-// K splits of the two-blocks-per-CU pipelined GEMM for more than kSplitTokens tokens: the least of the time
-// of its rounds (0.9 us per K chunk of a block alone on its CU, 1.64 us of two) and of the partials' write and
-// read, 2 us for the reduce launch where the call has none anyway.  512 tokens: the down projection's 48
-// blocks of 70 chunks 63.5 us, in 5 splits 21.5 us and its
-// reduce step 7.1 us (which carries the next RMSNorm + quantization, 5.2 us as a launch of its own).
-static int pipe_splits(const GemmArgs& a, int nkc, int row_tiles) {
+// K splits of the two-blocks-per-CU pipelined GEMM with blocks of `tok` tokens and `tiles` row tiles: the least
+// of the time of its rounds (`alone` us per K chunk of a block alone on its CU, `pair` of two) and of the
+// partials' write and read, 2 us for the reduce launch where the call has none anyway.
+static int pipe_splits(const GemmArgs& a, int tok, int tiles, double alone, double pair) {
   if (!a.part || a.out_dim > QWEN_QKV_ROWS) return 1;
-  const int blocks = (a.tokens + 63) / 64 * ((row_tiles + 15) / 16);
+  const int nkc = a.in_dim / kKChunk;
+  const int blocks = (a.tokens + tok - 1) / tok * ((a.out_dim / 16 + tiles - 1) / tiles);
   int best = 1;
   double cost = 0.0;
   for (int s = 1; s <= kMaxSplits; ++s) {
-    if (nkc % s != 0 || s * a.tokens > kSplitRows) continue;
+    if (nkc % s != 0 || (s > 1 && s * a.tokens > kSplitRows)) continue;
     const int n = blocks * s;
-    const double rounds = n <= 256 ? 0.9 : 1.64 * ((n + 511) / 512);
+    const double rounds = n <= 256 ? alone : pair * ((n + 511) / 512);
     const double c = rounds * (nkc / s) + (s > 1 || a.fuse != kFuseNone ? s * (double)a.tokens * a.out_dim * 8.0 / 4.5e6 : 0.0) +
                      (s > 1 && a.fuse == kFuseNone ? 2.0 : 0.0);
     if (s == 1 || c < cost) {
@@ -3907,13 +3941,11 @@ static int pipe_splits(const GemmArgs& a, int nkc, int row_tiles) {
   return best;
 }
 
-// Shape dispatch (the split-K workspace a.part, when given, holds kSplitRows x out_dim floats).  <= 16 tokens: direct-load kernel, 4-way in-block K split per row tile (many
+// Shape dispatch (the split-K workspace a.part, when given: splitk_bytes).  <= 16 tokens: direct-load kernel, 4-way in-block K split per row tile (many
 // small blocks, weights streamed once).  More tokens: the pipelined LDS kernel; projections whose
 // row tiles alone give fewer than ~256 blocks are also split over K across blocks (needs a.part).
 template <int EPI, bool DUAL>
 static void launch_gemm_epi(const GemmArgs& a, hipStream_t st) {
-  const int nkc = a.in_dim / kKChunk;
-  const int row_tiles = a.out_dim / 16;
   // The grouped SiLU·up code (gsx/gcorr read by the down projection, gsx_out/gcorr_out written by
   // gate/up) exists only in the skinny kernels: any other kernel would ignore it, reading the zero
   // limb sums or leaving the code stale.  Such a call either takes the skinny kernel or fails.
@@ -3936,13 +3968,14 @@ static void launch_gemm_epi(const GemmArgs& a, hipStream_t st) {
     return;
   }
   if constexpr (!DUAL && EPI == kEpiStore) {
-    if (a.fuse == kFuseRopePrefill) {
-      if (a.tokens <= kSkinnyTokens || a.out_dim != QWEN_QKV_ROWS || a.seq_len <= 0 || a.past < 0 || !a.rope ||
-          !a.k_cache || !a.v_cache)
-        throw std::runtime_error("prefill RoPE epilogue: more than 64 tokens of the [q | k | v] projection");
-      // one head per block while two-head blocks (8 per 64 tokens) do not fill the CUs: 512 tokens 17.2 -> 12.0 us
+    if (a.fuse == kFuseRopePrefill || a.fuse == kFuseQkvRope) {
+      const bool where = a.fuse == kFuseQkvRope ? a.pos != nullptr : !a.pos && a.seq_len > 0 && a.past >= 0;
+      if (a.tokens <= kSkinnyTokens || a.out_dim != QWEN_QKV_ROWS || !where || !a.rope || !a.k_cache || !a.v_cache)
+        throw std::runtime_error("RoPE epilogue: more than 64 tokens of the [q | k | v] projection");
+      // one head and 32 tokens per block while two-head blocks of 64 tokens (8 per 64 tokens) do not fill the CUs
+      // (512 tokens: 17.2 us; one head of 64 tokens 12.0 us, of 32 tokens 8.9 us)
       if ((a.tokens + 63) / 64 * 8 <= 256)
-        launch_gemm_pipe_t<4, 2, 2, EPI, DUAL, 1, 2, true, true>(a, 1, st);
+        launch_gemm_pipe_t<2, 2, 2, EPI, DUAL, 1, 2, false, true>(a, 1, st);
       else
         launch_gemm_pipe_t<4, 4, 2, EPI, DUAL, 1, 2, true, true>(a, 1, st);
       return;
@@ -3951,30 +3984,20 @@ static void launch_gemm_epi(const GemmArgs& a, hipStream_t st) {
   // Many tokens (prefill): 4-wave blocks of 64 tokens with two LDS stages (64 KiB), two blocks per
   // CU.  Measured against one 8-wave block of 128 tokens with three stages (144 KiB) per CU at 16,384
   // tokens: gate/up 0.94-0.98 -> 0.79 ms, down 0.38-0.40 -> 0.34 ms, QKV 111-118 -> 97-100 us.
-  if (a.tokens > kSplitTokens) {
-    if constexpr (DUAL)
+  if constexpr (DUAL) {
+    // (32-token blocks up to 256 tokens, 4 layers: 200 tokens 482 -> 413 us against one 64-token block with
+    // four LDS stages per CU; 330 tokens 483 -> 497 us)
+    if (a.tokens > kSplitTokens)
       launch_gemm_pipe_t<4, 2, 2, EPI, DUAL, 1, 2, true>(a, 1, st);
     else
-      launch_gemm_pipe_t<4, 4, 2, EPI, DUAL, 1, 2, true>(a, pipe_splits(a, nkc, row_tiles), st);
-    return;
-  }
-  if constexpr (DUAL) {
-    if (a.tokens <= 64)
-      launch_gemm_pipe_t<4, 1, 4, EPI, DUAL>(a, 1, st);
-    else
-      launch_gemm_pipe_t<4, 2, 4, EPI, DUAL>(a, 1, st);
+      launch_gemm_pipe_t<2, 2, 2, EPI, DUAL, 1, 2>(a, 1, st);
   } else {
-    if (a.tokens <= 64) {
-      const int blocks = (row_tiles + 3) / 4;
-      const int splits = a.part ? split_for(nkc, (256 + blocks - 1) / blocks) : 1;
-      launch_gemm_pipe_t<4, 1, 4, EPI, DUAL>(a, splits, st);  // a.part holds >= kSplitTokens rows
-    } else {
-      const int token_tiles = (a.tokens + 63) / 64;
-      const int blocks = token_tiles * ((row_tiles + 15) / 16);
-      const int splits =
-          (a.part && a.tokens <= kSplitTokens && blocks < 256) ? split_for(nkc, (256 + blocks - 1) / blocks) : 1;
-      launch_gemm_pipe_t<4, 4, 4, EPI, DUAL>(a, splits, st);
-    }
+    // blocks of 32 tokens x 128 rows while 64 x 256 would give few (4 layers: 100 tokens 385 -> 352 us, 512
+    // tokens 544 -> 525 us; 2000 tokens 392 -> 402 us a layer)
+    if (a.tokens <= kPrefillFuseTokens)
+      launch_gemm_pipe_t<2, 2, 2, EPI, DUAL, 1, 2>(a, pipe_splits(a, 32, 8, 0.5, 0.7), st);
+    else
+      launch_gemm_pipe_t<4, 4, 2, EPI, DUAL, 1, 2, true>(a, pipe_splits(a, 64, 16, 0.9, 1.64), st);
   }
 }
 
@@ -4130,8 +4153,8 @@ void launch_rope_qkv(float* qkv, int qkv_stride, const int* pos, int seq_len, in
                      rope, k_cache, v_cache, seq_stride);
 }
 
-constexpr int kAttnMinChunk = 64;
-constexpr int kAttnSoftSplits = 24;
+constexpr int kRaggedFrom = kSkinnyTokens, kRaggedMost = 1024;  // batches split by their own lengths
+constexpr int kAttnSoftSplits = 24, kAttnSoftSplitsLong = 48;
 
 AttnDecodePlan plan_attn_decode(int batch, int max_keys, int cus) {
   // co-resident blocks of attn_decode_kernel on the current device (CUs x blocks per CU)
@@ -4145,15 +4168,23 @@ AttnDecodePlan plan_attn_decode(int batch, int max_keys, int cus) {
   }();
   // at most 3 co-resident blocks per CU: the KV stream runs faster at 12 than at 16 waves per CU
   const int slots = (cus > 0 && cus < dev_slots.x ? cus : dev_slots.x) * (dev_slots.y < 3 ? dev_slots.y : 3);
+  if (batch > kRaggedFrom && batch <= kRaggedMost) {
+    const int blocks = max(slots / QWEN_KV_HEADS, batch / 2 + 128);
+    const int most = min(kAttnSoftSplits, max(4, 4096 / batch));  // bounds the partials' workspace
+    return AttnDecodePlan{most, 0, blocks};
+  }
   int nsplit = slots / (QWEN_KV_HEADS * (batch > 0 ? batch : 1));
   nsplit = nsplit < 1 ? 1 : (nsplit > kAttnMaxSplits ? kAttnMaxSplits : nsplit);
   int chunk = (max_keys + nsplit - 1) / nsplit;
   // Small batches cannot fill the device: each extra split then costs more in the merge (one memory
   // round trip per 8 splits) than it saves.  Measured on MI355X (batch 1-16, 544 and 4128 keys):
-  // at least 64 keys per split and at most 24 splits.
-  chunk = max(chunk, max(kAttnMinChunk, (max_keys + kAttnSoftSplits - 1) / kAttnSoftSplits));
+  // at least 64 keys per split and at most 24 splits; one sequence of more than 1536 keys (two of more
+  // than 4096) gains from 48 (4 layers, one sequence: 9001 keys 226 -> 201 us, 3000 keys 187 -> 180 us; two
+  // of 5000 to 9000 keys 297 -> 286 us; four of 8000 298 -> 310 us).
+  const int soft = batch <= 1 || (batch == 2 && max_keys > 4096) ? kAttnSoftSplitsLong : kAttnSoftSplits;
+  chunk = max(chunk, max(kAttnMinChunk, (max_keys + soft - 1) / soft));
   chunk = (chunk + 15) & ~15;  // whole 16-key tiles
-  return AttnDecodePlan{(max_keys + chunk - 1) / chunk, chunk};
+  return AttnDecodePlan{(max_keys + chunk - 1) / chunk, chunk, 0};
 }
 
 void launch_zero_u32(unsigned* p, int n, hipStream_t st) {
@@ -4162,12 +4193,25 @@ void launch_zero_u32(unsigned* p, int n, hipStream_t st) {
 
 void launch_attn_decode(const float* qkv, int qkv_stride, const float* k_cache, const float* v_cache,
                         size_t seq_stride, const int* pos, int batch, int max_keys, const AttnDecodePlan& plan,
-                        float* part, float2* pml, float* ctx, int8_t* xq, float* sx, int* sums, hipStream_t st) {
-  hipLaunchKernelGGL(attn_decode_kernel, dim3(plan.nsplit, QWEN_KV_HEADS, batch), dim3(256), 0, st, qkv, qkv_stride,
-                     k_cache, v_cache, seq_stride, pos, plan.chunk, max_keys, part, pml);
-  if (xq)
-    hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(batch), dim3(256), 0, st, part, pml, pos, 1, 0, plan.nsplit,
-                       plan.chunk, max_keys, ctx, xq, sx, sums);
+                        float* part, float2* pml, int* budget, float* ctx, int8_t* xq, float* sx, int* sums,
+                        hipStream_t st) {
+  if (plan.ragged_blocks > 0) {
+    // sum_s ceil(n_s / C) <= sum n_s / C + batch <= (blocks - batch / 2) + batch
+    const RaggedArgs ra{batch, plan.ragged_blocks, plan.nsplit, budget};
+    const unsigned grid = 2u * (unsigned)(plan.ragged_blocks - batch / 2 + batch);
+    hipLaunchKernelGGL(attn_decode_ragged_kernel, dim3(grid), dim3(256), 0, st, qkv, qkv_stride, k_cache, v_cache,
+                       seq_stride, pos, max_keys, part, pml, ra);
+  } else {
+    hipLaunchKernelGGL(attn_decode_kernel, dim3(plan.nsplit, QWEN_KV_HEADS, batch), dim3(256), 0, st, qkv, qkv_stride,
+                       k_cache, v_cache, seq_stride, pos, plan.chunk, max_keys, part, pml);
+  }
+  if (!xq) return;
+  if (plan.ragged_blocks > 0)
+    hipLaunchKernelGGL(attn_ragged_merge_kernel, dim3(batch), dim3(256), 0, st, part, pml, pos, plan.nsplit, max_keys,
+                       budget, ctx, xq, sx, sums);
+  else
+    hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(batch), dim3(256), 0, st, part, pml, pos, plan.nsplit, plan.chunk,
+                       max_keys, ctx, xq, sx, sums);
 }
 
 size_t attn_prefill_workspace_bytes(int keys, int nseq) {
@@ -4181,7 +4225,7 @@ AttnPrefillPlan plan_attn_prefill(int S, int past, int nseq) {
   double cost = 0.0;
   // The time in tiles of a block alone on its CU (1.2 us): its tiles and about 4 for its start and end while
   // every block has a CU; two blocks on a CU take 2.2 times as long per tile, and the CUs share what there
-  // is.  The partials' write and read add 100 KB per block.
+  // is.  The partials' write and read add 100 KB per block, the merge about 2 to the quantization it replaces.
   for (int n = 1; n <= kAttnMaxSplits && n <= ntiles; ++n) {
     const int tps = (ntiles + n - 1) / n;
     if (n > 1 && tps == (ntiles + n - 2) / (n - 1)) continue;  // same tiles per split: fewer splits
@@ -4194,7 +4238,7 @@ AttnPrefillPlan plan_attn_prefill(int S, int past, int nseq) {
     total *= 2.0 * nseq;
     blocks *= 2.0 * nseq;
     const double alone = tps + 4.0, share = 1.1 * (total + 4.0 * blocks) / 256.0;
-    const double c = (blocks <= 256.0 ? alone : share > 2.2 * alone ? share : 2.2 * alone) + (n > 1 ? blocks * 0.03 : 0.0);
+    const double c = (blocks <= 256.0 ? alone : share > 2.2 * alone ? share : 2.2 * alone) + (n > 1 ? 2.0 + blocks * 0.03 : 0.0);
     if (n == 1 || c < cost) {
       cost = c;
       best = AttnPrefillPlan{n, tps};
@@ -4215,9 +4259,8 @@ void launch_attn_prefill(const float* qkv, int qkv_stride, const float* k_cache,
   if (plan.nsplit > 1) {
     hipLaunchKernelGGL(attn_prefill_tiles_kernel<true>, grid, block, 0, st, qkv, qkv_stride, kv_tiles, S, past, ctx,
                        plan.nsplit, plan.tps, part, pml);
-    hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(nseq * S), dim3(256), 0, st, part, pml,
-                       static_cast<const int*>(nullptr), S, past, plan.nsplit, plan.tps * kPfKeys, keys,
-                       static_cast<float*>(nullptr), xq, sx, sums);
+    hipLaunchKernelGGL(attn_prefill_merge_kernel, dim3(nseq * S), dim3(256), 0, st, part, pml, S, past, plan.nsplit,
+                       plan.tps * kPfKeys, xq, sx, sums);
     return;
   }
   hipLaunchKernelGGL(attn_prefill_tiles_kernel<false>, grid, block, 0, st, qkv, qkv_stride, kv_tiles, S, past, ctx, 1, 0,

@@ -94,6 +94,7 @@ struct qwen_hip_model {
     float* gsx;     //   scales and offset terms
     int* gcorr;
     const int* zero_sums;  // kSkinnyTokens x (0, 0): the limb sums of code whose offsets are applied per group
+    int* budget;           // ragged decode attention: keys per block
     float* gmax;           // one token: max |SiLU.up| of each 16-row block of the gate/up projection
   };
   // Fixed region at the start of the workspace: the zero limb sums, zeroed once per workspace buffer
@@ -117,13 +118,14 @@ struct qwen_hip_model {
     const size_t o_tmp = take(tokens * QWEN_INTERMEDIATE * 4u);
     const size_t o_part = take(batch * QWEN_Q_HEADS * nsplit * QWEN_HEAD_DIM * 4u);
     const size_t o_pml = take(batch * QWEN_Q_HEADS * nsplit * 8u);
-    const size_t o_splitk = take(splitk_bytes(kQkvRows));
+    const size_t o_splitk = take(splitk_bytes(kQkvRows, tokens));
     const size_t o_kvt = take(kvt_bytes);
     const size_t gtok = tokens < (size_t)kSkinnyTokens ? tokens : (size_t)kSkinnyTokens;
     const size_t o_gxq = take(xq_bytes(gtok, QWEN_INTERMEDIATE));
     const size_t o_gsx = take(gtok * (QWEN_INTERMEDIATE / 64) * 4u);
     const size_t o_gcorr = take(gtok * (QWEN_INTERMEDIATE / 64) * 4u);
     const size_t o_gmax = take((QWEN_INTERMEDIATE / 16) * 4u);
+    const size_t o_budget = take(4u);
     char* b = static_cast<char*>(ws.get(off));
     if (ws.generation != zero_sums_ready) {  // fresh buffer: zero the sums once
       launch_zero_u32(reinterpret_cast<unsigned*>(b + o_zs), (int)(2 * kSkinnyTokens), stream);
@@ -136,7 +138,8 @@ struct qwen_hip_model {
               reinterpret_cast<float*>(b + o_part), reinterpret_cast<float2*>(b + o_pml),
               reinterpret_cast<float*>(b + o_splitk), reinterpret_cast<uint8_t*>(b + o_kvt),
               reinterpret_cast<int8_t*>(b + o_gxq), reinterpret_cast<float*>(b + o_gsx), reinterpret_cast<int*>(b + o_gcorr),
-              reinterpret_cast<const int*>(b + o_zs), reinterpret_cast<float*>(b + o_gmax)};
+              reinterpret_cast<const int*>(b + o_zs), reinterpret_cast<int*>(b + o_budget),
+              reinterpret_cast<float*>(b + o_gmax)};
   }
 
   Ws carve_prefill(size_t tokens, int nseq, int keys, const AttnPrefillPlan& plan) {
@@ -297,14 +300,14 @@ struct qwen_hip_model {
       const FastLayer& f = fast[l];
       float* kc = kc0 + (size_t)i * ls;
       float* vc = vc0 + (size_t)i * ls;
-      // With at most kSplitTokens sequences, RoPE + KV append and the two RMSNorm + quantize steps
-      // run inside the split-K reduce kernels of the QKV, O and down projections.
+      // RoPE + KV append run inside the Q/K/V projection; with at most kSplitTokens sequences the two
+      // RMSNorm + quantize steps run inside the split-K reduce kernels of the O and down projections.
       // (one sequence with the attention fused: the first layer's RMSNorm and quantization run in the
       // Q/K/V blocks' prologue instead)
       if ((i == 0 && !fuse_attn) || !fused)
         launch_norm_quant(hidden, QWEN_HIDDEN, B, QWEN_HIDDEN, f.ln, kNormDecode, w.xq, w.sx, w.sums, nullptr,
                           stream);
-      if (fused) {
+      {
         GemmArgs fq{};
         fq.fuse = kFuseQkvRope;
         fq.pos = pos;
@@ -344,14 +347,11 @@ struct qwen_hip_model {
           gemm(w, B, QWEN_HIDDEN, (int)kQkvRows, f.qkv, f.sw_qkv, f.b_qkv, w.qkv, kQkvRows, kEpiStore, nullptr,
                nullptr, nullptr, 0, 0, &fq);
         }
-      } else {
-        gemm(w, B, QWEN_HIDDEN, (int)kQkvRows, f.qkv, f.sw_qkv, f.b_qkv, w.qkv, kQkvRows, kEpiStore);
-        launch_rope_qkv(w.qkv, (int)kQkvRows, pos, 1, 0, max_keys, B, rope_decode, kc, vc, ss, stream);
       }
       // one sequence: the attention leaves its split partials, merged by every block of the O projection
       if (!fuse_attn)
-        launch_attn_decode(w.qkv, (int)kQkvRows, kc, vc, ss, pos, B, max_keys, plan, w.part, w.pml, nullptr,
-                           one ? nullptr : w.xq, w.sx, w.sums, stream);
+        launch_attn_decode(w.qkv, (int)kQkvRows, kc, vc, ss, pos, B, max_keys, plan, w.part, w.pml, w.budget,
+                           nullptr, one ? nullptr : w.xq, w.sx, w.sums, stream);
       GemmArgs fn{};
       fn.fuse = kFuseNormQuant;
       fn.norm = kNormDecode;
@@ -841,7 +841,8 @@ int qwen_hip_model_time_kernel(qwen_hip_model* m, int kernel, int layer, int rep
         case QWEN_KERNEL_ATTN_DECODE:
           // the partials launch alone (without xq no merge follows): the kernel the roofline covers
           launch_attn_decode(w.qkv, (int)kQkvRows, c.k_cache + la, c.v_cache + la, c.seq_stride, c.positions,
-                             c.batch, c.max_keys, plan, w.part, w.pml, nullptr, nullptr, w.sx, w.sums, m->stream);
+                             c.batch, c.max_keys, plan, w.part, w.pml, w.budget, nullptr, nullptr, w.sx, w.sums,
+                             m->stream);
           break;
         case QWEN_KERNEL_GEMM_GATE_UP:
           m->gemm(w, T, QWEN_HIDDEN, QWEN_INTERMEDIATE, f.gate, f.sw_gate, nullptr, w.tmp, QWEN_INTERMEDIATE,
