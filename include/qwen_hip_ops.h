@@ -42,8 +42,8 @@ int qwen_hip_fast_quantize_rows(const float* x, int rows, int n, int8_t* xq, flo
  * INT4 matrix w in the reference layout ([out_dim][in_dim] nibbles, the even flat index in the low
  * nibble; llm_memory_layout.h weight segments) with per-row scales sw [out_dim] and an optional bias
  * [out_dim] (null for none).  out_dim a multiple of 16, in_dim a multiple of 128 and <= 8960.  The
- * kernel is chosen by shape exactly as inside the model (<= 64 tokens: the skinny decode GEMMs; up to
- * 256: the pipelined GEMM with a cross-block K split; more: the pipelined GEMM with two blocks per CU).
+ * kernel is chosen by shape exactly as inside the model (<= 64 tokens: the skinny decode GEMMs; more: the
+ * pipelined GEMM in blocks of 32 or 64 tokens, with a cross-block K split where its blocks would be few).
  * Allocates its own workspace (repacked weights, activation code, split partials) and synchronizes
  * `stream` before returning. */
 int qwen_hip_fast_project(const uint8_t* w, const float* sw, const float* bias, int out_dim, int in_dim,

@@ -1,5 +1,5 @@
 """FAST prefill at the token counts where its launches change form: the K splits of the O and down projections,
-one or two heads per Q/K/V block, and the attention's key splits (a query tile's keys over several blocks,
+one or two heads per Q/K/V block, the skinny kernels' 64 tokens with several sequences in a tile, and the attention's key splits (a query tile's keys over several blocks,
 splits past a query's last key, a single query tile behind a long history).  Every size against ORDERED on the
 same input, per tensor within 1e-3 of its maximum (the FAST contract of the layer)."""
 
@@ -36,7 +36,8 @@ def run(model, mode, x, batch, seq, past, seed, layers):
 
 
 @pytest.mark.parametrize("batch,seq,past", [(1, 65, 0), (1, 130, 0), (3, 90, 0), (1, 257, 0), (1, 400, 0), (2, 400, 33),
-                                            (1, 1025, 0), (1, 5, 3000), (1, 16, 700), (1, 33, 2047), (2, 70, 1500)])
+                                            (1, 1025, 0), (1, 5, 3000), (1, 16, 700), (1, 33, 2047), (2, 70, 1500),
+                                            (1, 1, 0), (1, 17, 0), (3, 21, 5), (64, 1, 7), (1, 64, 0)])
 def test_layer_against_ordered(model, batch, seq, past):
     import torch
 

@@ -68,13 +68,13 @@ constexpr int kMaxQuantRow = 8960;  // widest activation row that is quantized
 constexpr int kAttnMaxSplits = 64;  // most KV splits of one decode-attention sequence
 constexpr int kNormNone = 0, kNormDecode = 1, kNormPrefill = 2;
 constexpr int kEpiStore = 0, kEpiSiluMul = 1, kEpiResidual = 2;
-// Epilogues fused into the split-K reduce kernel (GEMMs of at most kSplitTokens tokens):
-//   kFuseQkvRope:   [q|k|v] rows + bias, decode RoPE of q and k, K/V cache append (kEpiStore);
+// Fused into the split-K reduce kernel:
 //   kFuseNormQuant: the finished row (kEpiStore, or kEpiResidual after bf16 rounding) is RMS-normalized
 //                   with norm_w and quantized into xq_out / sx_out / sums_out for the next projection.
-// Fused into the epilogue of the pipelined GEMM (more than kSkinnyTokens tokens):
-//   kFuseRopePrefill: [q|k|v] rows + bias, prefill RoPE of q (in place in y) and k, K/V cache append;
-//                     token t is sequence t / seq_len at position past + t % seq_len.
+// Fused into the epilogue of the [q|k|v] projection (kEpiStore, + bias): RoPE of q (in place in y) and k, K/V
+// cache append.
+//   kFuseQkvRope:     decode, token t is sequence t at position pos[t];
+//   kFuseRopePrefill: token t is sequence t / seq_len at position past + t % seq_len.
 constexpr int kFuseNone = 0, kFuseQkvRope = 1, kFuseNormQuant = 2, kFuseRopePrefill = 3;
 
 // Bytes of the two-limb code of `rows` activation rows of width n.
@@ -213,10 +213,6 @@ bool launch_gemm_i8_prea(const GemmArgs& a, const AttnMergeArgs& am, hipStream_t
 bool launch_gemm_i8_attn(const GemmArgs& a, const AttnFuseArgs& af, hipStream_t st);
 bool launch_gemm_i8_pre_attn(const GemmArgs& a, const GemmArgs& pre, int pre_splits, const AttnFuseArgs& af,
                              hipStream_t st);
-// Decode (pos given): token t is sequence t at position pos[t].  Prefill (pos null): token t is
-// sequence t / seq_len at position past + t % seq_len.  Positions outside [0, limit) are skipped.
-void launch_rope_qkv(float* qkv, int qkv_stride, const int* pos, int seq_len, int past, int limit, int tokens,
-                     const float* rope, float* k_cache, float* v_cache, size_t seq_stride, hipStream_t st);
 // Decode attention split: nsplit blocks of `chunk` keys (a multiple of 16) per sequence and KV
 // head, sized so that one launch fills the device once.  Workspace: part [batch][12][nsplit][128]
 // floats, pml [batch][12][nsplit] (m, l) pairs.  launch_attn_decode leaves the split partials there,

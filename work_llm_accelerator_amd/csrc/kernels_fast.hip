@@ -713,7 +713,7 @@ constexpr int kIntSumMaxK = 8192;
 // untouched): wave w of a block (RTW = 4: 2 heads,
 // 16 row tiles) holds row tiles h*8 + 2*(w & 1) + {0, 1} and the same + 4 of head h = w >> 1, so that
 // tiles r and r + 2 hold the rotation pairs (p, p + 64) of one head and the epilogue rotates q and k and
-// appends K/V to the cache, as rope_qkv_kernel does after a plain store.  RTW = 2 (one head per block, for
+// appends K/V to the cache.  RTW = 2 (one head per block, for
 // launches whose 2-head blocks would leave CUs idle): wave w holds row tiles w and w + 4 of its head.
 template <int NT, int RTW, int NBUF, int EPI, bool DUAL, int TW, int WPE = 1, bool OWN = false, bool ROPE = false,
           int EF = 0>
@@ -1577,7 +1577,7 @@ __device__ __forceinline__ void kernarg_lines_wait(const KernargLines<BYTES>& l)
 
 template <int RTW, bool DUAL, int EPI, int NKC, bool ROPE, int KSW, bool PRE, int PRE_EPI = kEpiStore,
           bool PRE_QUANT = false, bool PRE_ATTN = false, bool GRP = false, bool ATTN = false, bool NEWKEY = false,
-          bool KW = false, int MKF = 16, int HOT_KB = 0, int HOT_IN = 0, int HOT_OUT = 0>
+          bool KW = false, int MKF = 16, int HOT_KB = 0, int HOT_IN = 0, int HOT_OUT = 0, bool SEQ = false>
 __device__ __forceinline__ void gemm_skinny_body(const GemmArgs& a, int tt_count, int rg_count, int splits,
                                                  const GemmArgs& pre, int pre_splits,
                                                  const AttnMergeArgs& am = AttnMergeArgs{},
@@ -1723,7 +1723,10 @@ __device__ __forceinline__ void gemm_skinny_body(const GemmArgs& a, int tt_count
   // decode position of this lane's token (RoPE epilogue), loaded with the weights
   // (ATTN, one token: read through the scalar cache once the weights are in flight, in issue_kv: a
   // vector load here made the compiler wait for every load in flight before its first use)
-  int P = ROPE && !ATTN ? pos_p[min(tok0 + col, n_tok - 1)] : 0;
+  // (SEQ, a prefill: token t is token t % seq_len of sequence t / seq_len, at position past + t % seq_len)
+  static_assert(!SEQ || (ROPE && !ATTN && !kMade), "SEQ: the [q | k | v] projection of a prefill");
+  int seq = tok0 + col;
+  int P = ROPE && !ATTN && !SEQ ? pos_p[min(tok0 + col, n_tok - 1)] : 0;
   // RoPE cos/sin of pairs p = 16*wave + 4g + q, q < 4, at position P (ATTN: loaded in issue_kv, ahead
   // of the K/V rows; otherwise after the slice barrier, in flight during the MFMAs)
   float4 rc = make_float4(1.0f, 1.0f, 1.0f, 1.0f), rs = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -1977,6 +1980,11 @@ __device__ __forceinline__ void gemm_skinny_body(const GemmArgs& a, int tt_count
   // Loaded by every lane at a clamped position (rope_in selects their use): under a run-time
   // condition the load is a branch, whose join waited for every load in flight, the weight stream
   // included, before the first MFMA.
+  if constexpr (SEQ) {
+    const int t = min(tok0 + col, n_tok - 1);
+    seq = t / a.seq_len;
+    P = a.past + t - seq * a.seq_len;
+  }
   const bool rope_in = ROPE && P >= 0 && P < a.limit;
   if constexpr (ROPE && !ATTN) load_rope();
   v4i accH[RTW][D], accL[RTW][D];
@@ -2300,7 +2308,7 @@ __device__ __forceinline__ void gemm_skinny_body(const GemmArgs& a, int tt_count
     if (head < QWEN_Q_HEADS) {
       dst = a.y + (size_t)tok * a.y_stride + head * QWEN_HEAD_DIM + p0;
     } else if (rope_in) {
-      const size_t cache_row = (size_t)tok * a.seq_stride + (size_t)P * QWEN_KV_WIDTH;
+      const size_t cache_row = (size_t)seq * a.seq_stride + (size_t)P * QWEN_KV_WIDTH;
       dst = head < QWEN_Q_HEADS + QWEN_KV_HEADS
                 ? a.k_cache + cache_row + (head - QWEN_Q_HEADS) * QWEN_HEAD_DIM + p0
                 : a.v_cache + cache_row + (head - QWEN_Q_HEADS - QWEN_KV_HEADS) * QWEN_HEAD_DIM + p0;
@@ -2438,13 +2446,13 @@ gemm_skinny_kernel(GemmArgs a, int tt_count, int rg_count, int splits) {
 // The same for the model's shapes (IN -> OUT) with the operands of the first loads preloaded (HotArgs:
 // the activation code, the weights, the up matrix or group scales, the positions, offset terms or
 // grouped code's scales out, then the counts).
-template <int RTW, bool DUAL, int EPI, int NKC, bool ROPE, int KSW, bool GRP, int IN, int OUT>
+template <int RTW, bool DUAL, int EPI, int NKC, bool ROPE, int KSW, bool GRP, int IN, int OUT, bool SEQ = false>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(3)))
 gemm_skinny_hot_kernel(const void* p0, const void* p1, const void* p2, const void* p3, int tokens, int tt_count,
                        int rg_count, int splits, GemmArgs a) {
   constexpr int kKb = kernarg_bytes<const void*, const void*, const void*, const void*, int, int, int, int, GemmArgs>();
   gemm_skinny_body<RTW, DUAL, EPI, NKC, ROPE, KSW, false, kEpiStore, false, false, GRP, false, false, false, 16, kKb,
-                   IN, OUT>(a, tt_count, rg_count, splits, a, 0, AttnMergeArgs{}, AttnFuseArgs{},
+                   IN, OUT, SEQ>(a, tt_count, rg_count, splits, a, 0, AttnMergeArgs{}, AttnFuseArgs{},
                             HotArgs{p0, p1, p2, p3, nullptr, nullptr, tokens});
 }
 
@@ -3009,47 +3017,6 @@ __global__ void __launch_bounds__(128) reduce_norm_quant_pair_hot_kernel(const v
   else
     reduce_norm_quant_row_zb<EPI, 5, decltype(issue)&, 2, true>(a, splits, tok, nullptr, 256, nullptr, nullptr, true,
                                                                 issue, hot);
-}
-
-// ---------------------------------------------------------------------------------------------
-// RoPE of q (in place) and k, plus the K/V cache append, for rows of a fused [q | k | v] buffer
-// (qkv_stride floats per token).  Decode: token b is sequence b at position pos[b].  Prefill:
-// token t is sequence t / seq_len at position t % seq_len.  rope: [position][cos 64 | sin 64].
-// Positions outside [0, limit) are skipped (limit = the cache rows the caller sized).
-// grid = tokens, block = 64 (one rotation pair per thread).
-// ---------------------------------------------------------------------------------------------
-__global__ void __launch_bounds__(64) rope_qkv_kernel(float* __restrict__ qkv, int qkv_stride,
-                                                      const int* __restrict__ pos, int seq_len, int past, int limit,
-                                                      const float* __restrict__ rope, float* __restrict__ k_cache,
-                                                      float* __restrict__ v_cache, size_t seq_stride) {
-  const int t = blockIdx.x;
-  const int p = threadIdx.x;
-  const int seq = pos ? t : t / seq_len;
-  const int P = pos ? pos[t] : past + t % seq_len;
-  if (P < 0 || P >= limit) return;  // position outside the cache rows the caller sized
-  const float c = rope[(size_t)P * 128 + p];
-  const float sn = rope[(size_t)P * 128 + 64 + p];
-  float* row = qkv + (size_t)t * qkv_stride;
-#pragma unroll
-  for (int h = 0; h < QWEN_Q_HEADS; ++h) {
-    float* hp = row + h * QWEN_HEAD_DIM;
-    const float e = hp[p], od = hp[p + 64];
-    hp[p] = e * c - od * sn;
-    hp[p + 64] = od * c + e * sn;
-  }
-  const float* kr = row + QWEN_HIDDEN;
-  const float* vr = row + QWEN_HIDDEN + QWEN_KV_WIDTH;
-  float* kc = k_cache + (size_t)seq * seq_stride + (size_t)P * QWEN_KV_WIDTH;
-  float* vc = v_cache + (size_t)seq * seq_stride + (size_t)P * QWEN_KV_WIDTH;
-#pragma unroll
-  for (int h = 0; h < QWEN_KV_HEADS; ++h) {
-    const int base = h * QWEN_HEAD_DIM;
-    const float e = kr[base + p], od = kr[base + p + 64];
-    kc[base + p] = e * c - od * sn;
-    kc[base + p + 64] = od * c + e * sn;
-    vc[base + p] = vr[base + p];
-    vc[base + p + 64] = vr[base + p + 64];
-  }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -3857,7 +3824,7 @@ static void launch_gemm_pipe_t(const GemmArgs& a, int splits, hipStream_t st) {
 // Skinny GEMMs for at most kSkinnyTokens tokens with in_dim 1536 (12 K chunks in one block) or 8960
 // (5 splits of 14 chunks, finished by the reduce step).  Returns false for other shapes.
 
-template <int RTW, bool DUAL, int EPI, int NKC, bool ROPE, int KSW = 1, bool GRP = false>
+template <int RTW, bool DUAL, int EPI, int NKC, bool ROPE, int KSW = 1, bool GRP = false, bool SEQ = false>
 static void launch_skinny_t(const GemmArgs& a, int rg_count, int splits, hipStream_t st) {
   // the grouped code's per-group sums are only finished by the split-K partial epilogue
   if (GRP && splits <= 1) throw std::runtime_error("grouped-code GEMM needs the split-K partial epilogue");
@@ -3870,13 +3837,17 @@ static void launch_skinny_t(const GemmArgs& a, int rg_count, int splits, hipStre
   if (kIn > 0 && a.in_dim == kIn && a.out_dim == kOut && splits * NKC * kKChunk == kIn) {
     const void* p2 = GRP ? (const void*)a.gsx : DUAL ? (const void*)a.wp2 : nullptr;
     const void* p3 = GRP ? (const void*)a.gcorr : ROPE ? (const void*)a.pos : DUAL ? (const void*)a.gsx_out : nullptr;
-    hipLaunchKernelGGL((gemm_skinny_hot_kernel<RTW, DUAL, EPI, NKC, ROPE, KSW, GRP, kIn, kOut>), dim3(blocks),
+    hipLaunchKernelGGL((gemm_skinny_hot_kernel<RTW, DUAL, EPI, NKC, ROPE, KSW, GRP, kIn, kOut, SEQ>), dim3(blocks),
                        dim3(256 * KSW), 0, st, (const void*)a.xq, (const void*)a.wp, p2, p3, a.tokens, tt, rg_count,
                        splits, a);
     return;
   }
-  hipLaunchKernelGGL((gemm_skinny_kernel<RTW, DUAL, EPI, NKC, ROPE, KSW, GRP>), dim3(blocks), dim3(256 * KSW), 0, st, a,
-                     tt, rg_count, splits);
+  if constexpr (SEQ) {
+    throw std::runtime_error("prefill RoPE epilogue: the [q | k | v] projection only");
+  } else {
+    hipLaunchKernelGGL((gemm_skinny_kernel<RTW, DUAL, EPI, NKC, ROPE, KSW, GRP>), dim3(blocks), dim3(256 * KSW), 0, st,
+                       a, tt, rg_count, splits);
+  }
 }
 
 template <int EPI, bool DUAL>
@@ -3892,6 +3863,18 @@ static bool launch_skinny(const GemmArgs& a, hipStream_t st) {
         launch_skinny_t<2, false, kEpiStore, 12, true, 2>(a, row_tiles / 8, 1, st);
       else
         launch_skinny_t<2, false, kEpiStore, 12, true, 1>(a, row_tiles / 8, 1, st);
+      return true;
+    }
+    if (!DUAL && EPI == kEpiStore && a.fuse == kFuseRopePrefill) {
+      // a prefill of at most 64 tokens: the decode batch's kernel with the positions of a prefill.  With the
+      // reduce steps and the grouped code that follow (prefill_fast) 9 launches per layer instead of 12: 47
+      // tokens over 4 layers 304 -> 272 us
+      if (a.out_dim != QWEN_QKV_ROWS || a.pos || a.seq_len <= 0 || a.past < 0 || !a.rope || !a.k_cache || !a.v_cache)
+        throw std::runtime_error("prefill RoPE epilogue: bad arguments");
+      if (a.tokens > 16)
+        launch_skinny_t<2, false, kEpiStore, 12, true, 2, false, true>(a, row_tiles / 8, 1, st);
+      else
+        launch_skinny_t<2, false, kEpiStore, 12, true, 1, false, true>(a, row_tiles / 8, 1, st);
       return true;
     }
     if (!DUAL && a.fuse != kFuseNone && !a.part) return false;
@@ -3941,9 +3924,10 @@ static int pipe_splits(const GemmArgs& a, int tok, int tiles, double alone, doub
   return best;
 }
 
-// Shape dispatch (the split-K workspace a.part, when given: splitk_bytes).  <= 16 tokens: direct-load kernel, 4-way in-block K split per row tile (many
-// small blocks, weights streamed once).  More tokens: the pipelined LDS kernel; projections whose
-// row tiles alone give fewer than ~256 blocks are also split over K across blocks (needs a.part).
+// Shape dispatch (the split-K workspace a.part, when given: splitk_bytes).  <= 64 tokens of the model's shapes: the
+// skinny kernels.  Other shapes of <= 16 tokens: direct-load kernel, 4-way in-block K split per row tile (many small
+// blocks, weights streamed once).  Else the pipelined LDS kernel, in blocks of 32 or 64 tokens, O and down also
+// split over K across blocks (pipe_splits; needs a.part).
 template <int EPI, bool DUAL>
 static void launch_gemm_epi(const GemmArgs& a, hipStream_t st) {
   // The grouped SiLU·up code (gsx/gcorr read by the down projection, gsx_out/gcorr_out written by
@@ -4145,12 +4129,6 @@ void launch_gemm_i8(const GemmArgs& a, int epi, hipStream_t st) {
     case kEpiResidual: launch_gemm_epi<kEpiResidual, false>(a, st); break;
     default: break;
   }
-}
-
-void launch_rope_qkv(float* qkv, int qkv_stride, const int* pos, int seq_len, int past, int limit, int tokens,
-                     const float* rope, float* k_cache, float* v_cache, size_t seq_stride, hipStream_t st) {
-  hipLaunchKernelGGL(rope_qkv_kernel, dim3(tokens), dim3(64), 0, st, qkv, qkv_stride, pos, seq_len, past, limit,
-                     rope, k_cache, v_cache, seq_stride);
 }
 
 constexpr int kRaggedFrom = kSkinnyTokens, kRaggedMost = 1024;  // batches split by their own lengths

@@ -441,7 +441,13 @@ struct qwen_hip_model {
     const Ws w = carve_prefill(T, B, past + S, plan);
     // Up to kPrefillFuseTokens tokens the RMSNorm + quantization that follow the O and down projections run in
     // the step that adds those projections' K splits (their 64-token tiles alone fill a fraction of the CUs).
-    const bool fused = T > kSkinnyTokens && T <= kPrefillFuseTokens;
+    // Up to kSkinnyTokens the SiLU·up rows go to the down projection in the grouped code, as a decode batch's.
+    const bool fused = T <= kPrefillFuseTokens;
+    const bool grouped = T <= kSkinnyTokens;
+    GemmArgs gq{};
+    gq.xq_out = w.gxq;
+    gq.gsx_out = w.gsx;
+    gq.gcorr_out = w.gcorr;
     GemmArgs fn{};
     fn.fuse = kFuseNormQuant;
     fn.norm = kNormPrefill;
@@ -455,23 +461,18 @@ struct qwen_hip_model {
       if (!fused || i == 0)
         launch_norm_quant(hidden, QWEN_HIDDEN, T, QWEN_HIDDEN, f.ln, kNormPrefill, w.xq, w.sx, w.sums, nullptr,
                           stream);
-      if (T > kSkinnyTokens) {
-        // RoPE of q and k and the K/V cache append in the Q/K/V projection's epilogue
-        GemmArgs fr{};
-        fr.fuse = kFuseRopePrefill;
-        fr.rope = rope_prefill;
-        fr.k_cache = kc;
-        fr.v_cache = vc;
-        fr.seq_stride = ss;
-        fr.seq_len = S;
-        fr.past = past;
-        fr.limit = past + S;
-        gemm(w, T, QWEN_HIDDEN, (int)kQkvRows, f.qkv, f.sw_qkv, f.b_qkv, w.qkv, kQkvRows, kEpiStore, nullptr, nullptr,
-             nullptr, 0, 0, &fr);
-      } else {
-        gemm(w, T, QWEN_HIDDEN, (int)kQkvRows, f.qkv, f.sw_qkv, f.b_qkv, w.qkv, kQkvRows, kEpiStore);
-        launch_rope_qkv(w.qkv, (int)kQkvRows, nullptr, S, past, past + S, T, rope_prefill, kc, vc, ss, stream);
-      }
+      // RoPE of q and k and the K/V cache append in the Q/K/V projection's epilogue
+      GemmArgs fr{};
+      fr.fuse = kFuseRopePrefill;
+      fr.rope = rope_prefill;
+      fr.k_cache = kc;
+      fr.v_cache = vc;
+      fr.seq_stride = ss;
+      fr.seq_len = S;
+      fr.past = past;
+      fr.limit = past + S;
+      gemm(w, T, QWEN_HIDDEN, (int)kQkvRows, f.qkv, f.sw_qkv, f.b_qkv, w.qkv, kQkvRows, kEpiStore, nullptr, nullptr,
+           nullptr, 0, 0, &fr);
       launch_attn_prefill(w.qkv, (int)kQkvRows, kc, vc, ss, S, past, B, w.kvt, plan, w.part, w.pml, w.ctx, w.xq, w.sx,
                           w.sums, stream);
       if (plan.nsplit == 1)
@@ -483,13 +484,21 @@ struct qwen_hip_model {
         launch_norm_quant(w.att, QWEN_HIDDEN, T, QWEN_HIDDEN, f.post_ln, kNormPrefill, w.xq, w.sx, w.sums, nullptr,
                           stream);
       gemm(w, T, QWEN_HIDDEN, QWEN_INTERMEDIATE, f.gate, f.sw_gate, nullptr, w.s, QWEN_INTERMEDIATE, kEpiSiluMul,
-           f.up, f.sw_up, nullptr, 0, 1);
-      launch_norm_quant(w.s, QWEN_INTERMEDIATE, T, QWEN_INTERMEDIATE, nullptr, kNormNone, w.xq, w.sx, w.sums,
-                        nullptr, stream);
+           f.up, f.sw_up, nullptr, 0, 1, grouped ? &gq : nullptr);
+      if (!grouped)
+        launch_norm_quant(w.s, QWEN_INTERMEDIATE, T, QWEN_INTERMEDIATE, nullptr, kNormNone, w.xq, w.sx, w.sums,
+                          nullptr, stream);
       const bool fuse_next = fused && i + 1 < count;  // the next layer's input RMSNorm + quantize
       fn.norm_w = fuse_next ? fast[first + i + 1].ln : nullptr;
-      gemm(w, T, QWEN_INTERMEDIATE, QWEN_HIDDEN, f.down, f.sw_down, nullptr, hidden, QWEN_HIDDEN, kEpiResidual,
-           nullptr, nullptr, w.att, round, 0, fuse_next ? &fn : nullptr);
+      GemmArgs da = args(w, T, QWEN_INTERMEDIATE, QWEN_HIDDEN, f.down, f.sw_down, nullptr, hidden, QWEN_HIDDEN,
+                         nullptr, nullptr, w.att, round, 0, fuse_next ? &fn : nullptr);
+      if (grouped) {  // the down partials carry the per-group offsets: the reduce step gets zero sums
+        da.xq = w.gxq;
+        da.gsx = w.gsx;
+        da.gcorr = w.gcorr;
+        da.sums = w.zero_sums;
+      }
+      launch_gemm_i8(da, kEpiResidual, stream);
     }
     QWEN_HIP(hipGetLastError());
   }
