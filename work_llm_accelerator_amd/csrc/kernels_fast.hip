@@ -708,7 +708,7 @@ constexpr int kIntSumMaxK = 8192;
 // its accumulator slot 0, and the wave runs half of that slot's MFMAs before the chunk's barrier (its
 // own loads have landed by its own wait), so waves that reach the barrier late are absorbed by matrix
 // work instead of stalling the others.  Slot n holds token tile (wv + n) mod 4.
-// ROPE (the fused [q | k | v] projection of a prefill, kFuseRopePrefill, or of a decode batch, kFuseQkvRope:
+// ROPE (the fused [q | k | v] projection of a prefill, kFuseRopePrefill; BATCH: of a decode batch, kFuseQkvRope:
 // token t at position pos[t] of sequence t, a position outside [0, limit) leaving q unrotated and the cache
 // untouched): wave w of a block (RTW = 4: 2 heads,
 // 16 row tiles) holds row tiles h*8 + 2*(w & 1) + {0, 1} and the same + 4 of head h = w >> 1, so that
@@ -716,7 +716,7 @@ constexpr int kIntSumMaxK = 8192;
 // appends K/V to the cache.  RTW = 2 (one head per block, for
 // launches whose 2-head blocks would leave CUs idle): wave w holds row tiles w and w + 4 of its head.
 template <int NT, int RTW, int NBUF, int EPI, bool DUAL, int TW, int WPE = 1, bool OWN = false, bool ROPE = false,
-          int EF = 0>
+          int EF = 0, bool BATCH = false>
 __global__ void __launch_bounds__(256 * TW) __attribute__((amdgpu_waves_per_eu(WPE))) gemm_i8_pipe_kernel(GemmArgs a) {
   static_assert(!OWN || (TW == 1 && NT == 4), "own tile first: each of the 4 waves loads one token tile");
   static_assert(!ROPE || ((RTW == 4 || RTW == 2) && TW == 1 && !DUAL && EPI == kEpiStore), "prefill RoPE: 1 or 2 heads per block");
@@ -940,8 +940,8 @@ __global__ void __launch_bounds__(256 * TW) __attribute__((amdgpu_waves_per_eu(W
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
           const int tc = min(tok[n], a.tokens - 1);
-          seqn[n] = a.pos ? tc : tc / a.seq_len;
-          Pn[n] = a.pos ? a.pos[tc] : a.past + tc % a.seq_len;
+          seqn[n] = BATCH ? tc : tc / a.seq_len;
+          Pn[n] = BATCH ? a.pos[tc] : a.past + tc % a.seq_len;
           const int Pc = min(max(Pn[n], 0), a.limit - 1);
           cs[n] = *reinterpret_cast<const float4*>(a.rope + (size_t)Pc * 128 + p);
           sn[n] = *reinterpret_cast<const float4*>(a.rope + (size_t)Pc * 128 + 64 + p);
@@ -949,7 +949,7 @@ __global__ void __launch_bounds__(256 * TW) __attribute__((amdgpu_waves_per_eu(W
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
           const bool in = Pn[n] >= 0 && Pn[n] < a.limit;
-          if (tok[n] >= a.tokens || (!in && head >= QWEN_Q_HEADS)) continue;
+          if (tok[n] >= a.tokens || (!in && (!BATCH || head >= QWEN_Q_HEADS))) continue;
           float e[4], od[4];
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
@@ -962,7 +962,7 @@ __global__ void __launch_bounds__(256 * TW) __attribute__((amdgpu_waves_per_eu(W
           float lo[4], hi[4];
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            const bool plain = head >= QWEN_Q_HEADS + QWEN_KV_HEADS || !in;
+            const bool plain = head >= QWEN_Q_HEADS + QWEN_KV_HEADS || (BATCH && !in);
             lo[q] = plain ? e[q] : e[q] * c4[q] - od[q] * s4[q];
             hi[q] = plain ? od[q] : od[q] * c4[q] + e[q] * s4[q];
           }
@@ -3021,7 +3021,7 @@ __global__ void __launch_bounds__(128) reduce_norm_quant_pair_hot_kernel(const v
 
 // ---------------------------------------------------------------------------------------------
 // Decode attention on the fp32 matrix cores, split over the KV length; the split merge and the
-// O-projection input quantization follow in attn_decode_merge_kernel (qwen_decode_attention_kernel.cpp:113-162 semantics:
+// O-projection input quantization follow in attn_merge_kernel (qwen_decode_attention_kernel.cpp:113-162 semantics:
 // s_t = (q . k_t) * 0.08838834764831845f over keys 0..pos, softmax, ctx = sum_t p_t v_t; here with
 // an online softmax, reordered sums and __expf).
 // grid = (nsplit, 2 KV heads, batch), block = 256 (4 waves).  Block (split c, KV head kvh, sequence
@@ -3144,12 +3144,13 @@ __device__ __forceinline__ int ragged_chunk(int n, int budget) {
   return ((n + k - 1) / k + 15) & ~15;
 }
 
+// (One kernel template and no shared device function: inlined into two kernels, the body was optimized in another
+// order, and a layer of 64 sequences of 4096 keys took 1.3 us more of 143.)
 template <bool RAGGED>
-__device__ __forceinline__ void attn_decode_body(const float* __restrict__ qkv, int qkv_stride,
-                                                 const float* __restrict__ k_cache, const float* __restrict__ v_cache,
-                                                 size_t seq_stride, const int* __restrict__ pos, int chunk, int max_keys,
-                                                 float* __restrict__ part, float2* __restrict__ pml,
-                                                 const RaggedArgs& ra) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+attn_decode_kernel(const float* __restrict__ qkv, int qkv_stride, const float* __restrict__ k_cache,
+                   const float* __restrict__ v_cache, size_t seq_stride, const int* __restrict__ pos, int chunk,
+                   int max_keys, float* __restrict__ part, float2* __restrict__ pml, RaggedArgs ra) {
   // (the leading 14 argument dwords, through max_keys, are preloaded: the first loads wait for nothing;
   // the segment's other lines are requested at entry and waited for once the first tile is in flight)
   const auto klines = kernarg_lines_issue<
@@ -3322,19 +3323,6 @@ __device__ __forceinline__ void attn_decode_body(const float* __restrict__ qkv, 
   }
 }
 
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
-attn_decode_kernel(const float* __restrict__ qkv, int qkv_stride, const float* __restrict__ k_cache,
-                   const float* __restrict__ v_cache, size_t seq_stride, const int* __restrict__ pos, int chunk,
-                   int max_keys, float* __restrict__ part, float2* __restrict__ pml) {
-  attn_decode_body<false>(qkv, qkv_stride, k_cache, v_cache, seq_stride, pos, chunk, max_keys, part, pml, RaggedArgs{});
-}
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
-attn_decode_ragged_kernel(const float* __restrict__ qkv, int qkv_stride, const float* __restrict__ k_cache,
-                          const float* __restrict__ v_cache, size_t seq_stride, const int* __restrict__ pos,
-                          int max_keys, float* __restrict__ part, float2* __restrict__ pml, RaggedArgs ra) {
-  attn_decode_body<true>(qkv, qkv_stride, k_cache, v_cache, seq_stride, pos, 0, max_keys, part, pml, ra);
-}
-
 // The split merge of attn_decode_kernel's partials, one block per sequence (RAGGED: the splits follow from
 // *budget), or of the split prefill attention's, one block per token (token b at position past + b % seq_len):
 // per head the merge
@@ -3346,11 +3334,11 @@ attn_decode_ragged_kernel(const float* __restrict__ qkv, int qkv_stride, const f
 // at most 8 splits need one memory round trip.
 constexpr int kMergeDecode = 0, kMergeRagged = 1, kMergePrefill = 2;
 template <int MODE>
-__device__ __forceinline__ void attn_merge_body(const float* __restrict__ part, const float2* __restrict__ pml,
-                                                const int* __restrict__ pos, int nsplit, int chunk, int max_keys,
-                                                float* __restrict__ ctx, int8_t* __restrict__ xq, float* __restrict__ sx,
-                                                int* __restrict__ sums, int seq_len, int past,
-                                                const int* __restrict__ budget) {
+__global__ void __launch_bounds__(256) attn_merge_kernel(const float* __restrict__ part, const float2* __restrict__ pml,
+                                                         const int* __restrict__ pos, int nsplit, int chunk, int max_keys,
+                                                         float* __restrict__ ctx, int8_t* __restrict__ xq,
+                                                         float* __restrict__ sx, int* __restrict__ sums, int seq_len,
+                                                         int past, const int* __restrict__ budget) {
   constexpr int kF4 = QWEN_HIDDEN / 4;  // float4 columns of the row
   __shared__ __align__(16) float row[QWEN_HIDDEN];         // the context row
   __shared__ float ml[QWEN_Q_HEADS * kAttnMaxSplits * 2];  // (m, l), then merge weights in place
@@ -3409,29 +3397,6 @@ __device__ __forceinline__ void attn_merge_body(const float* __restrict__ part, 
   }
   __syncthreads();
   quantize_row_lds(row, QWEN_HIDDEN, xq + (size_t)b * (2 * QWEN_HIDDEN), sx + b, sums + 2 * b, red_f, red_i);
-}
-
-__global__ void __launch_bounds__(256) attn_decode_merge_kernel(const float* __restrict__ part,
-                                                                const float2* __restrict__ pml,
-                                                                const int* __restrict__ pos, int nsplit, int chunk,
-                                                                int max_keys, float* __restrict__ ctx,
-                                                                int8_t* __restrict__ xq, float* __restrict__ sx,
-                                                                int* __restrict__ sums) {
-  attn_merge_body<kMergeDecode>(part, pml, pos, nsplit, chunk, max_keys, ctx, xq, sx, sums, 1, 0, nullptr);
-}
-__global__ void __launch_bounds__(256) attn_ragged_merge_kernel(const float* __restrict__ part,
-                                                                const float2* __restrict__ pml,
-                                                                const int* __restrict__ pos, int nsplit, int max_keys,
-                                                                const int* __restrict__ budget, float* __restrict__ ctx,
-                                                                int8_t* __restrict__ xq, float* __restrict__ sx,
-                                                                int* __restrict__ sums) {
-  attn_merge_body<kMergeRagged>(part, pml, pos, nsplit, 0, max_keys, ctx, xq, sx, sums, 1, 0, budget);
-}
-__global__ void __launch_bounds__(256) attn_prefill_merge_kernel(const float* __restrict__ part,
-                                                                 const float2* __restrict__ pml, int seq_len, int past,
-                                                                 int nsplit, int chunk, int8_t* __restrict__ xq,
-                                                                 float* __restrict__ sx, int* __restrict__ sums) {
-  attn_merge_body<kMergePrefill>(part, pml, nullptr, nsplit, chunk, 0, nullptr, xq, sx, sums, seq_len, past, nullptr);
 }
 
 __global__ void zero_u32_kernel(unsigned* __restrict__ p, int n) {
@@ -3543,7 +3508,7 @@ __global__ void __launch_bounds__(256) kv_bf16_tiles_kernel(const float* __restr
 // grid = (ceil(S/16), 2, nseq) with query tiles longest first, block = 448.
 // SPLIT: few query tiles leave most CUs idle, so the key tiles of a query tile go to several blocks of tps
 // tiles each (grid.z = nseq * nsplit); a block leaves its queries' unnormalized rows and (max, sum) in
-// part[token][head][split][128], pml[token][head][split] for attn_prefill_merge_kernel, which also forms the
+// part[token][head][split][128], pml[token][head][split] for attn_merge_kernel, which also forms the
 // O projection's input code (one launch, as the quantization alone).  385 queries after 3000 keys (50 query
 // tiles): 131 -> 39 us and the merge 7 us
 // where the quantization took 5; 512 queries: 24.5 -> 11 us.
@@ -3794,7 +3759,8 @@ static void launch_reduce(const GemmArgs& a, int splits, hipStream_t st) {
   }
 }
 
-template <int NT, int RTW, int NBUF, int EPI, bool DUAL, int TW = 1, int WPE = 1, bool OWN = false, bool ROPE = false>
+template <int NT, int RTW, int NBUF, int EPI, bool DUAL, int TW = 1, int WPE = 1, bool OWN = false, bool ROPE = false,
+          bool BATCH = false>
 static void launch_gemm_pipe_t(const GemmArgs& a, int splits, hipStream_t st) {
   const int row_tiles = a.out_dim / 16;
   const int nblk = ((a.tokens + 16 * NT * TW - 1) / (16 * NT * TW)) * ((row_tiles + 4 * RTW - 1) / (4 * RTW));
@@ -3802,8 +3768,8 @@ static void launch_gemm_pipe_t(const GemmArgs& a, int splits, hipStream_t st) {
   // epilogue form: the int32 limb combination where in_dim allows it, and the SiLU the call asks for
   const bool int_sum = a.in_dim <= kIntSumMaxK;
   auto go = [&](auto ef) {
-    hipLaunchKernelGGL((gemm_i8_pipe_kernel<NT, RTW, NBUF, EPI, DUAL, TW, WPE, OWN, ROPE, decltype(ef)::value>), grid,
-                       dim3(256 * TW), 0, st, a);
+    hipLaunchKernelGGL((gemm_i8_pipe_kernel<NT, RTW, NBUF, EPI, DUAL, TW, WPE, OWN, ROPE, decltype(ef)::value, BATCH>),
+                       grid, dim3(256 * TW), 0, st, a);
   };
   if constexpr (EPI == kEpiSiluMul) {
     if (a.prefill_silu)
@@ -3958,10 +3924,17 @@ static void launch_gemm_epi(const GemmArgs& a, hipStream_t st) {
         throw std::runtime_error("RoPE epilogue: more than 64 tokens of the [q | k | v] projection");
       // one head and 32 tokens per block while two-head blocks of 64 tokens (8 per 64 tokens) do not fill the CUs
       // (512 tokens: 17.2 us; one head of 64 tokens 12.0 us, of 32 tokens 8.9 us)
-      if ((a.tokens + 63) / 64 * 8 <= 256)
+      const bool few = (a.tokens + 63) / 64 * 8 <= 256;
+      if (a.fuse == kFuseQkvRope) {
+        if (few)
+          launch_gemm_pipe_t<2, 2, 2, EPI, DUAL, 1, 2, false, true, true>(a, 1, st);
+        else
+          launch_gemm_pipe_t<4, 4, 2, EPI, DUAL, 1, 2, true, true, true>(a, 1, st);
+      } else if (few) {
         launch_gemm_pipe_t<2, 2, 2, EPI, DUAL, 1, 2, false, true>(a, 1, st);
-      else
+      } else {
         launch_gemm_pipe_t<4, 4, 2, EPI, DUAL, 1, 2, true, true>(a, 1, st);
+      }
       return;
     }
   }
@@ -4140,7 +4113,7 @@ AttnDecodePlan plan_attn_decode(int batch, int max_keys, int cus) {
     int dev = 0, per_cu = 0;
     hipDeviceProp_t prop;
     if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess) return int2{256, 4};
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, attn_decode_kernel, 256, 0) != hipSuccess || per_cu < 1)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, attn_decode_kernel<false>, 256, 0) != hipSuccess || per_cu < 1)
       per_cu = 1;
     return int2{prop.multiProcessorCount, per_cu};
   }();
@@ -4177,19 +4150,19 @@ void launch_attn_decode(const float* qkv, int qkv_stride, const float* k_cache, 
     // sum_s ceil(n_s / C) <= sum n_s / C + batch <= (blocks - batch / 2) + batch
     const RaggedArgs ra{batch, plan.ragged_blocks, plan.nsplit, budget};
     const unsigned grid = 2u * (unsigned)(plan.ragged_blocks - batch / 2 + batch);
-    hipLaunchKernelGGL(attn_decode_ragged_kernel, dim3(grid), dim3(256), 0, st, qkv, qkv_stride, k_cache, v_cache,
-                       seq_stride, pos, max_keys, part, pml, ra);
+    hipLaunchKernelGGL(attn_decode_kernel<true>, dim3(grid), dim3(256), 0, st, qkv, qkv_stride, k_cache, v_cache,
+                       seq_stride, pos, 0, max_keys, part, pml, ra);
   } else {
-    hipLaunchKernelGGL(attn_decode_kernel, dim3(plan.nsplit, QWEN_KV_HEADS, batch), dim3(256), 0, st, qkv, qkv_stride,
-                       k_cache, v_cache, seq_stride, pos, plan.chunk, max_keys, part, pml);
+    hipLaunchKernelGGL(attn_decode_kernel<false>, dim3(plan.nsplit, QWEN_KV_HEADS, batch), dim3(256), 0, st, qkv,
+                       qkv_stride, k_cache, v_cache, seq_stride, pos, plan.chunk, max_keys, part, pml, RaggedArgs{});
   }
   if (!xq) return;
   if (plan.ragged_blocks > 0)
-    hipLaunchKernelGGL(attn_ragged_merge_kernel, dim3(batch), dim3(256), 0, st, part, pml, pos, plan.nsplit, max_keys,
-                       budget, ctx, xq, sx, sums);
+    hipLaunchKernelGGL(attn_merge_kernel<kMergeRagged>, dim3(batch), dim3(256), 0, st, part, pml, pos, plan.nsplit, 0,
+                       max_keys, ctx, xq, sx, sums, 1, 0, budget);
   else
-    hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(batch), dim3(256), 0, st, part, pml, pos, plan.nsplit, plan.chunk,
-                       max_keys, ctx, xq, sx, sums);
+    hipLaunchKernelGGL(attn_merge_kernel<kMergeDecode>, dim3(batch), dim3(256), 0, st, part, pml, pos, plan.nsplit,
+                       plan.chunk, max_keys, ctx, xq, sx, sums, 1, 0, nullptr);
 }
 
 size_t attn_prefill_workspace_bytes(int keys, int nseq) {
@@ -4237,8 +4210,8 @@ void launch_attn_prefill(const float* qkv, int qkv_stride, const float* k_cache,
   if (plan.nsplit > 1) {
     hipLaunchKernelGGL(attn_prefill_tiles_kernel<true>, grid, block, 0, st, qkv, qkv_stride, kv_tiles, S, past, ctx,
                        plan.nsplit, plan.tps, part, pml);
-    hipLaunchKernelGGL(attn_prefill_merge_kernel, dim3(nseq * S), dim3(256), 0, st, part, pml, S, past, plan.nsplit,
-                       plan.tps * kPfKeys, xq, sx, sums);
+    hipLaunchKernelGGL(attn_merge_kernel<kMergePrefill>, dim3(nseq * S), dim3(256), 0, st, part, pml, nullptr,
+                       plan.nsplit, plan.tps * kPfKeys, 0, nullptr, xq, sx, sums, S, past, nullptr);
     return;
   }
   hipLaunchKernelGGL(attn_prefill_tiles_kernel<false>, grid, block, 0, st, qkv, qkv_stride, kv_tiles, S, past, ctx, 1, 0,
