@@ -45,10 +45,20 @@ struct CallScope {
     rt.arena.reset();
     rt.arena.reserve(arena_bytes);
   }
-  ~CallScope() { rt.arena.reset(); }
+  ~CallScope() {
+    // (a call that failed between its copies and its wait: the next one refills the pinned block)
+    if (rt.staging.pending() && hipStreamSynchronize(rt.stream) == hipSuccess) rt.staging.waited();
+    rt.staging.forget();
+    rt.arena.reset();
+  }
   hipStream_t st() const { return rt.stream; }
   Arena& A() { return rt.arena; }
-  void sync() { QWEN_HIP(hipStreamSynchronize(rt.stream)); }
+  Staging& small() { return rt.staging; }
+  void sync() {
+    QWEN_HIP(hipStreamSynchronize(rt.stream));
+    rt.staging.waited();
+    rt.staging.deliver();
+  }
 };
 
 bool any_null(std::initializer_list<const void*> ptrs) {
@@ -96,12 +106,15 @@ int decode_layer_host(const HostLayer& h, const float* x, int past, float* k_cac
     CallScope cs(decode_call_bytes(past));
     Arena& A = cs.A();
     const hipStream_t st = cs.st();
-    const DevLayer d = stage_layer(A, h, st);
-    const float* x_d = stage_in(A, x, QWEN_HIDDEN, st);
-    const int* pos_d = stage_in(A, &past, 1, st);
+    Staging& small = cs.small();
+    small.begin(A);
+    const float* x_d = small.add(x, QWEN_HIDDEN);
+    const int* pos_d = small.add(&past, 1);
     float rope_row[128];
     decode_rope_row_host(past, rope_row);
-    const float* rope_d = stage_in(A, rope_row, 128, st);
+    const float* rope_d = small.add(rope_row, 128);
+    const DevLayer d = stage_layer(A, small, h, st);
+    small.send(st);
     const size_t kv_n = (size_t)(past + 1) * QWEN_KV_WIDTH;
     float* kc_d = stage_in(A, k_cache, kv_n, st);
     float* vc_d = stage_in(A, v_cache, kv_n, st);
@@ -109,16 +122,16 @@ int decode_layer_host(const HostLayer& h, const float* x, int past, float* k_cac
     DecodeBatch b{1, pos_d, rope_d, true, kc_d, vc_d, 0, past + 1};
     run_decode_attention(d, x_d, b, att_d, A, st);
     const size_t row = (size_t)past * QWEN_KV_WIDTH;
-    copy_out(k_cache + row, kc_d + row, QWEN_KV_WIDTH, st);
-    copy_out(v_cache + row, vc_d + row, QWEN_KV_WIDTH, st);
-    if (att_host) copy_out(att_host, att_d, QWEN_HIDDEN, st);
+    small.collect(k_cache + row, kc_d + row, QWEN_KV_WIDTH * sizeof(float), st);
+    small.collect(v_cache + row, vc_d + row, QWEN_KV_WIDTH * sizeof(float), st);
+    if (att_host) small.collect(att_host, att_d, QWEN_HIDDEN * sizeof(float), st);
     if (!run_mlp || !mlp_args_ok) {
       cs.sync();
       return run_mlp ? QWEN_ERR_KERNEL : QWEN_OK;
     }
     float* out_d = A.alloc_n<float>(QWEN_HIDDEN);
     run_decode_mlp(d, att_d, 1, out_d, A, st);
-    copy_out(out, out_d, QWEN_HIDDEN, st);
+    small.collect(out, out_d, QWEN_HIDDEN * sizeof(float), st);
     cs.sync();
     return QWEN_OK;
   });
@@ -152,7 +165,9 @@ int qwen_decode_mlp_smoke_forward(const float* a, const float* post_ln, const ui
   h.post_ln = post_ln; h.gw = gw; h.uw = uw; h.dw = dw; h.gs = gs; h.us = us; h.ds = ds;
   return guarded([&]() -> int {
     CallScope cs(decode_call_bytes(0));
-    const DevLayer d = stage_layer(cs.A(), h, cs.st());
+    cs.small().begin(cs.A());
+    const DevLayer d = stage_layer(cs.A(), cs.small(), h, cs.st());
+    cs.small().send(cs.st());
     const float* a_d = stage_in(cs.A(), a, QWEN_HIDDEN, cs.st());
     float* out_d = cs.A().alloc_n<float>(QWEN_HIDDEN);
     run_decode_mlp(d, a_d, 1, out_d, cs.A(), cs.st());
@@ -252,7 +267,9 @@ int prefill_layer_host(const HostLayer& h, const float* x, int S, float* k_cache
     Arena& A = cs.A();
     const hipStream_t st = cs.st();
     const float* rope = cs.rt.prefill_rope(S);
-    const DevLayer d = stage_layer(A, h, st);
+    cs.small().begin(A);
+    const DevLayer d = stage_layer(A, cs.small(), h, st);
+    cs.small().send(st);
     const float* x_d = stage_in(A, x, (size_t)S * QWEN_HIDDEN, st);
     float* kc_d = A.alloc_n<float>((size_t)S * QWEN_KV_WIDTH);
     float* vc_d = A.alloc_n<float>((size_t)S * QWEN_KV_WIDTH);
@@ -315,7 +332,9 @@ int qwen_prefill_mlp_smoke_forward(const float* a, int S, int m_seq, int m_hidde
   h.post_ln = post_ln; h.gw = gw; h.uw = uw; h.dw = dw; h.gs = gs; h.us = us; h.ds = ds;
   return guarded([&]() -> int {
     CallScope cs(prefill_call_bytes(S));
-    const DevLayer d = stage_layer(cs.A(), h, cs.st());
+    cs.small().begin(cs.A());
+    const DevLayer d = stage_layer(cs.A(), cs.small(), h, cs.st());
+    cs.small().send(cs.st());
     const float* a_d = stage_in(cs.A(), a, (size_t)S * QWEN_HIDDEN, cs.st());
     float* out_d = cs.A().alloc_n<float>((size_t)S * QWEN_HIDDEN);
     run_prefill_mlp(d, a_d, S, out_d, cs.A(), cs.st());

@@ -72,6 +72,39 @@ void* Arena::alloc(size_t bytes) {
 }
 
 // ---------------------------------------------------------------------------------------------
+void Staging::begin(Arena& a) {
+  if (!host_) QWEN_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_), kBytes, hipHostMallocDefault));
+  dev_ = static_cast<char*>(a.alloc(kBytes));
+  used_ = 0;
+  n_results_ = 0;
+}
+
+size_t Staging::take(size_t bytes) {
+  const size_t at = (used_ + 255u) & ~size_t(255u);
+  if (at + bytes > kBytes) throw std::runtime_error("staging capacity exceeded");
+  used_ = at + bytes;
+  return at;
+}
+
+void Staging::send(hipStream_t st) {
+  pending_ = true;
+  QWEN_HIP(hipMemcpyAsync(dev_, host_, used_, hipMemcpyHostToDevice, st));
+}
+
+void Staging::collect(void* host, const void* dev, size_t bytes, hipStream_t st) {
+  if (n_results_ == 4) throw std::runtime_error("staging: too many results");
+  const size_t at = take(bytes);
+  pending_ = true;
+  QWEN_HIP(hipMemcpyAsync(host_ + at, dev, bytes, hipMemcpyDeviceToHost, st));
+  results_[n_results_++] = Result{host, at, bytes};
+}
+
+void Staging::deliver() {
+  for (int i = 0; i < n_results_; ++i) std::memcpy(results_[i].host, host_ + results_[i].at, results_[i].bytes);
+  n_results_ = 0;
+}
+
+// ---------------------------------------------------------------------------------------------
 Runtime& Runtime::get() {
   static Runtime* rt = new Runtime();  // never destroyed: HIP objects outlive static teardown
   return *rt;
@@ -126,9 +159,9 @@ const float* Runtime::decode_rope(int positions) {
 }
 
 // ---------------------------------------------------------------------------------------------
-size_t staged_layer_bytes() { return QWEN_LAYER_BYTES + 64u * 256u; }
+size_t staged_layer_bytes() { return QWEN_LAYER_BYTES + 64u * 256u + Staging::kBytes; }
 
-DevLayer stage_layer(Arena& a, const HostLayer& h, hipStream_t st) {
+DevLayer stage_layer(Arena& a, Staging& small, const HostLayer& h, hipStream_t st) {
   DevLayer d;
   d.qw = stage_in(a, h.qw, QWEN_Q_WEIGHT_BYTES, st);
   d.kw = stage_in(a, h.kw, QWEN_K_WEIGHT_BYTES, st);
@@ -137,18 +170,18 @@ DevLayer stage_layer(Arena& a, const HostLayer& h, hipStream_t st) {
   d.gw = stage_in(a, h.gw, QWEN_GATE_WEIGHT_BYTES, st);
   d.uw = stage_in(a, h.uw, QWEN_UP_WEIGHT_BYTES, st);
   d.dw = stage_in(a, h.dw, QWEN_DOWN_WEIGHT_BYTES, st);
-  d.ln = stage_in(a, h.ln, QWEN_HIDDEN, st);
-  d.post_ln = stage_in(a, h.post_ln, QWEN_HIDDEN, st);
-  d.qb = stage_in(a, h.qb, QWEN_HIDDEN, st);
-  d.kb = stage_in(a, h.kb, QWEN_KV_WIDTH, st);
-  d.vb = stage_in(a, h.vb, QWEN_KV_WIDTH, st);
-  d.qs = stage_in(a, h.qs, QWEN_HIDDEN, st);
-  d.ks = stage_in(a, h.ks, QWEN_KV_WIDTH, st);
-  d.vs = stage_in(a, h.vs, QWEN_KV_WIDTH, st);
-  d.os = stage_in(a, h.os, QWEN_HIDDEN, st);
-  d.gs = stage_in(a, h.gs, QWEN_INTERMEDIATE, st);
-  d.us = stage_in(a, h.us, QWEN_INTERMEDIATE, st);
-  d.ds = stage_in(a, h.ds, QWEN_HIDDEN, st);
+  d.ln = small.add(h.ln, QWEN_HIDDEN);
+  d.post_ln = small.add(h.post_ln, QWEN_HIDDEN);
+  d.qb = small.add(h.qb, QWEN_HIDDEN);
+  d.kb = small.add(h.kb, QWEN_KV_WIDTH);
+  d.vb = small.add(h.vb, QWEN_KV_WIDTH);
+  d.qs = small.add(h.qs, QWEN_HIDDEN);
+  d.ks = small.add(h.ks, QWEN_KV_WIDTH);
+  d.vs = small.add(h.vs, QWEN_KV_WIDTH);
+  d.os = small.add(h.os, QWEN_HIDDEN);
+  d.gs = small.add(h.gs, QWEN_INTERMEDIATE);
+  d.us = small.add(h.us, QWEN_INTERMEDIATE);
+  d.ds = small.add(h.ds, QWEN_HIDDEN);
   return d;
 }
 
