@@ -124,7 +124,7 @@ struct GemmArgs {
   float* y_raw;         // kEpiResidual: optional copy of the output before bf16 rounding
   int round_bf16;       // kEpiResidual: round the output to bf16 (driver rounding)
   int prefill_silu;     // kEpiSiluMul: 1 = approx_exp SiLU (prefill), 0 = expf SiLU (decode)
-  float* part;          // optional fp32 workspace for K splits across blocks: [splits][tokens][out]
+  float* part;          // optional workspace for K splits across blocks: [splits][tokens][out] words
   int fuse;             // kFuse*: epilogue of the reduce kernel (needs part)
   // kFuseQkvRope (token t is sequence t at position pos[t]; positions outside [0, limit) are skipped)
   const int* pos;
@@ -139,6 +139,8 @@ struct GemmArgs {
   int8_t* xq_out;
   float* sx_out;
   int* sums_out;
+  const int* zero_sums; // kFuseNormQuant, O of at most 64 tokens: optional zeros [tokens][2]; given, the
+                        // partial is the finished value (zero point off before its rounding, a prefill's)
   int defer_reduce;     // kFuseNormQuant, one token: write the partials only; the next projection's
                         // blocks finish the row (launch_gemm_i8_pre)
   int seq_len, past;    // kFuseRopePrefill (with rope, k_cache, v_cache, seq_stride, limit)

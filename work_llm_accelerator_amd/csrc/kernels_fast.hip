@@ -652,9 +652,12 @@ __global__ void __launch_bounds__(256) gemm_i8_kernel(GemmArgs a) {
 // Every vector-memory instruction of the loop is one of these loads, issued in chunk order, so
 // `s_waitcnt vmcnt(n)` with n = loads issued after chunk i is exactly "chunk i has landed"; a
 // barrier then makes every wave's part visible and frees the buffer refilled next.
-// gridDim.z > 1 splits the K chunks over blocks: each block writes fp32 partials
-// sw*sx*(256*sumH + sumL) of its chunks to a.part[z][tok][row], and gemm_splitk_reduce_kernel adds
-// them in z order, applies the -8*sum(X) correction and the epilogue.
+// gridDim.z > 1 splits the K chunks over blocks: each block writes the int32 sums 256*sumH + sumL of its
+// chunks to a.part[z][tok][row], and the reduce step adds them, takes off the zero point 8*sum(X), rounds
+// once and applies the epilogue: the unsplit kernel's values whatever the split (a single split before a
+// fused reduce step writes the finished sum in fp32).  Scaled fp32 partials that still hold the zero point
+// would be rounded relative to it: on rows of one sign (8960 inputs, 7 splits) 9e-6 of the result's norm
+// instead of 2e-8.  Times with either are within 1% (a layer of 65 to 1340 tokens).
 // grid = (ceil(tokens/(16*NT)), ceil(row_tiles/(4*RTW)), splits), block = 256.
 // ---------------------------------------------------------------------------------------------
 template <int VMCNT>
@@ -703,6 +706,11 @@ constexpr int kRasterGroup = 8;  // token tiles per raster group of the pipeline
 constexpr int kEfPrefillSilu = 1;
 constexpr int kEfIntSum = 2;
 constexpr int kIntSumMaxK = 8192;
+// Inputs whose sum of u X (0 <= u <= 15, |X| <= 32512) fits int32; wider K splits (two of the down
+// projection's 8960 inputs) run ZOFF, whose sums of q X fit.
+constexpr int kIntPartK = 34 * kKChunk;
+static_assert((long long)kIntPartK * 15 * kQuantMax < (1ll << 31), "int32 partials");
+static_assert((long long)(kMaxQuantRow / 2) * 8 * kQuantMax < (1ll << 31), "int32 partials without the zero point");
 
 // OWN (one token group of 4 tiles, TW = 1, NT = 4): the token tile a wave loads itself (tile wv) is
 // its accumulator slot 0, and the wave runs half of that slot's MFMAs before the chunk's barrier (its
@@ -715,8 +723,12 @@ constexpr int kIntSumMaxK = 8192;
 // tiles r and r + 2 hold the rotation pairs (p, p + 64) of one head and the epilogue rotates q and k and
 // appends K/V to the cache.  RTW = 2 (one head per block, for
 // launches whose 2-head blocks would leave CUs idle): wave w holds row tiles w and w + 4 of its head.
+// ZOFF (K splits wider than kIntPartK): the block takes its own split's zero point off its partials, from the
+// limb sums of its tokens over the split, which its waves add up beside the MFMAs (a tile and both limbs each,
+// or two waves per tile and one limb each).  A layer of 1200 tokens: 1 us more than with fp32 partials; with the
+// weights unpacked as q instead, 4 us.
 template <int NT, int RTW, int NBUF, int EPI, bool DUAL, int TW, int WPE = 1, bool OWN = false, bool ROPE = false,
-          int EF = 0, bool BATCH = false>
+          int EF = 0, bool BATCH = false, bool ZOFF = false>
 __global__ void __launch_bounds__(256 * TW) __attribute__((amdgpu_waves_per_eu(WPE))) gemm_i8_pipe_kernel(GemmArgs a) {
   static_assert(!OWN || (TW == 1 && NT == 4), "own tile first: each of the 4 waves loads one token tile");
   static_assert(!ROPE || ((RTW == 4 || RTW == 2) && TW == 1 && !DUAL && EPI == kEpiStore), "prefill RoPE: 1 or 2 heads per block");
@@ -820,6 +832,18 @@ __global__ void __launch_bounds__(256 * TW) __attribute__((amdgpu_waves_per_eu(W
         for (int n = 0; n < NT; ++n) accH[d][r][n] = accL[d][r][n] = v4i{0, 0, 0, 0};
   };
 
+  // ZOFF: limb sums of the wave's share (OWN: tile wv, both limbs; else tile wv & 1, limb wv >> 1)
+  static_assert(!ZOFF || (TW == 1 && !DUAL && !ROPE && (OWN || NT == 2)), "ZOFF: four waves' shares");
+  __shared__ int zs[ZOFF ? TOK : 1][2];
+  int zsum[2] = {0, 0};
+  auto add_limbs = [](int& sum, const v4i& x, const v4i& y) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      sum = __builtin_amdgcn_sdot4(x[i], 0x01010101, sum, false);
+      sum = __builtin_amdgcn_sdot4(y[i], 0x01010101, sum, false);
+    }
+  };
+
   // One chunk: the stage (xst, wst) holds it; (xnx, wnx) is the stage the next issue refills.
   auto chunk = [&](uint8_t* xst, uint8_t* wst, uint8_t* xnx, uint8_t* wnx) {
     // exactly NBUF-2 chunks were issued after this one: waiting for all but their loads means it has
@@ -884,6 +908,10 @@ __global__ void __launch_bounds__(256 * TW) __attribute__((amdgpu_waves_per_eu(W
 #pragma unroll
         for (int q = 0; q < 4; ++q) bx[1][q] = lds_read_b128(xo[q] + slot_off(1));
         mfma_slot(0, cur, D * RTW / 2, D * RTW);
+        if constexpr (ZOFF) {
+          add_limbs(zsum[0], cur[0], cur[1]);
+          add_limbs(zsum[1], cur[2], cur[3]);
+        }
         continue;
       }
       if (n + 1 < NT) {
@@ -895,10 +923,16 @@ __global__ void __launch_bounds__(256 * TW) __attribute__((amdgpu_waves_per_eu(W
       }
       if (n == 0) unpack_weights();
       mfma_slot(n, cur, 0, D * RTW);
+      if (ZOFF && !OWN && n == (wv & 1)) {
+        if (wv < 2)
+          add_limbs(zsum[0], cur[0], cur[1]);
+        else
+          add_limbs(zsum[0], cur[2], cur[3]);
+      }
     }
   };
 
-  const bool partial = gridDim.z > 1 || (!DUAL && a.fuse != kFuseNone);  // a reduce kernel finishes
+  const bool partial = ZOFF || gridDim.z > 1 || (!DUAL && a.fuse != kFuseNone);  // a reduce kernel finishes
   // Epilogue.  Every operand load is issued before the first use, so the wave waits for memory once
   // rather than once per (row tile, token tile); token columns past the last token read the last
   // token's values and store nothing.
@@ -912,8 +946,8 @@ __global__ void __launch_bounds__(256 * TW) __attribute__((amdgpu_waves_per_eu(W
       const int tc = min(tok[n], a.tokens - 1);
       sxv[n] = a.sx[tc];
       const int2 sm = *reinterpret_cast<const int2*>(a.sums + 2 * tc);
-      sh8[n] = 8 * sm.x;
-      sl8[n] = 8 * sm.y;
+      sh8[n] = 8 * (ZOFF ? zs[tok[n] - tok0][0] : sm.x);
+      sl8[n] = 8 * (ZOFF ? zs[tok[n] - tok0][1] : sm.y);
     }
     float sw[RTW][4], sw2[RTW][4], bias[RTW][4];
 #pragma unroll
@@ -1013,12 +1047,17 @@ __global__ void __launch_bounds__(256 * TW) __attribute__((amdgpu_waves_per_eu(W
       for (int n = 0; n < NT; ++n) {
         float out[4];
         if (partial) {
+          if (tok[n] >= a.tokens) continue;
+          float* dst = a.part + ((size_t)blockIdx.z * a.tokens + tok[n]) * a.out_dim + row0;
+          if (!ZOFF && gridDim.z == 1) {
+            *reinterpret_cast<float4*>(dst) =
+                make_float4(dequant(0, r, n, 0), dequant(0, r, n, 1), dequant(0, r, n, 2), dequant(0, r, n, 3));
+          } else {
+            int t[4];
 #pragma unroll
-          for (int q = 0; q < 4; ++q)
-            out[q] = ((float)accH[0][r][n][q] * 256.0f + (float)accL[0][r][n][q]) * sxv[n] * sw[r][q];
-          if (tok[n] < a.tokens)
-            *reinterpret_cast<float4*>(a.part + ((size_t)blockIdx.z * a.tokens + tok[n]) * a.out_dim + row0) =
-                make_float4(out[0], out[1], out[2], out[3]);
+            for (int q = 0; q < 4; ++q) t[q] = (int)(((uint32_t)accH[0][r][n][q] << 8) + (uint32_t)accL[0][r][n][q] - (ZOFF ? c8[n] : 0u));
+            *reinterpret_cast<int4*>(dst) = make_int4(t[0], t[1], t[2], t[3]);
+          }
           continue;
         }
 #pragma unroll
@@ -1056,6 +1095,22 @@ __global__ void __launch_bounds__(256 * TW) __attribute__((amdgpu_waves_per_eu(W
     }
   }
   wait_vmcnt<0>();  // the trailing reloads land before the wave moves on
+  if constexpr (ZOFF) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      zsum[i] += __shfl_xor(zsum[i], 16, 64);
+      zsum[i] += __shfl_xor(zsum[i], 32, 64);
+    }
+    if (g == 0) {
+      if (OWN) {
+        zs[wv * 16 + col][0] = zsum[0];
+        zs[wv * 16 + col][1] = zsum[1];
+      } else {
+        zs[(wv & 1) * 16 + col][wv >> 1] = zsum[0];
+      }
+    }
+    __syncthreads();
+  }
   epilogue();
 }
 
@@ -1077,10 +1132,10 @@ struct NoIssue {
   __device__ void operator()() const {}
 };
 
-// Elementwise pieces of the reduce step: the split sum plus zero-point correction, residual or bias,
-// optional y_raw / y stores and bf16 rounding of elements row0 .. row0 + 3; the sum of squares of
-// four elements in double; the RMSNorm scaling.
-template <int EPI>
+// Elementwise pieces of the reduce step: the split sum plus zero-point correction (EXACT: the exact sum
+// times the token's scale `corr` and the row scale), residual or bias, optional y_raw / y stores and bf16
+// rounding of elements row0 .. row0 + 3; the sum of squares of four elements in double; the RMSNorm scaling.
+template <int EPI, bool EXACT = false>
 __device__ __forceinline__ float4 rnq_combine(const GemmArgs& a, int tok, int row0, float4 acc, float4 sw, float4 ad,
                                               double corr, bool write_y) {
   const float s4[4] = {sw.x, sw.y, sw.z, sw.w};
@@ -1089,7 +1144,7 @@ __device__ __forceinline__ float4 rnq_combine(const GemmArgs& a, int tok, int ro
   float out[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const float val = p4[q] + (float)(corr * (double)s4[q]);
+    const float val = EXACT ? p4[q] * (float)corr * s4[q] : p4[q] + (float)(corr * (double)s4[q]);
     out[q] = EPI == kEpiResidual ? d4[q] + val : val + d4[q];
   }
   if (EPI == kEpiResidual && a.y_raw && write_y)
@@ -1133,7 +1188,11 @@ template <int EPI, class Issue = NoIssue>
 __device__ __forceinline__ void reduce_norm_quant_row(const GemmArgs& a, int splits, int tok, int8_t* xq_row,
                                                       int chunk_stride, float* sx_out, int* sums_out, bool write_y,
                                                       Issue&& issue = Issue{});
-template <int EPI, int ZB, class Issue, int W = 1, bool HOT = false>
+// The partials of the pipelined GEMM: the sum of all splits fits int32 with its zero point (in_dim at most
+// kIntPartK), or only that of two of five splits, or of three of seven or more.
+constexpr int kExactNarrow = 1, kExactWide = 2;
+static_assert(kMaxQuantRow / 5 * 2 <= kIntPartK && kMaxQuantRow / 7 * 3 <= kIntPartK, "int32 groups of splits");
+template <int EPI, int ZB, class Issue, int W = 1, bool HOT = false, int EXACT = 0>
 __device__ __forceinline__ void reduce_norm_quant_row_zb(const GemmArgs& a, int splits, int tok, int8_t* xq_row,
                                                          int chunk_stride, float* sx_out, int* sums_out, bool write_y,
                                                          Issue&& issue, const HotArgs& hot = HotArgs{});
@@ -1577,7 +1636,8 @@ __device__ __forceinline__ void kernarg_lines_wait(const KernargLines<BYTES>& l)
 
 template <int RTW, bool DUAL, int EPI, int NKC, bool ROPE, int KSW, bool PRE, int PRE_EPI = kEpiStore,
           bool PRE_QUANT = false, bool PRE_ATTN = false, bool GRP = false, bool ATTN = false, bool NEWKEY = false,
-          bool KW = false, int MKF = 16, int HOT_KB = 0, int HOT_IN = 0, int HOT_OUT = 0, bool SEQ = false>
+          bool KW = false, int MKF = 16, int HOT_KB = 0, int HOT_IN = 0, int HOT_OUT = 0, bool SEQ = false,
+          bool FIN = false>
 __device__ __forceinline__ void gemm_skinny_body(const GemmArgs& a, int tt_count, int rg_count, int splits,
                                                  const GemmArgs& pre, int pre_splits,
                                                  const AttnMergeArgs& am = AttnMergeArgs{},
@@ -2246,9 +2306,11 @@ __device__ __forceinline__ void gemm_skinny_body(const GemmArgs& a, int tt_count
   const bool partial = splits > 1 || (!DUAL && !ROPE && a.fuse != kFuseNone);
   if (partial) {
     // PRE_ATTN over a range of heads: the range has its own scale and limb sums, so its partial takes
-    // its own offset correction (the reduce step then adds the partials with a zero correction)
+    // its own offset correction (the reduce step then adds the partials with a zero correction); so does
+    // FIN, whose one split is the whole sum: the value the plain epilogue forms
+    static_assert(!FIN || (!kMade && !GRP && NKC * kKChunk == QWEN_HIDDEN), "FIN: one K group");
     constexpr bool kOwnCorr = PRE_ATTN && NKC * kKChunk < QWEN_HIDDEN;
-    const int ch8 = kOwnCorr ? 8 * pre_tot.x : 0, cl8 = kOwnCorr ? 8 * pre_tot.y : 0;
+    const int ch8 = kOwnCorr ? 8 * pre_tot.x : FIN ? 8 * sh_l : 0, cl8 = kOwnCorr ? 8 * pre_tot.y : FIN ? 8 * sl_l : 0;
 #pragma unroll
     for (int r = 0; r < RTW; ++r) {
       if (!ok[r]) continue;
@@ -2446,13 +2508,14 @@ gemm_skinny_kernel(GemmArgs a, int tt_count, int rg_count, int splits) {
 // The same for the model's shapes (IN -> OUT) with the operands of the first loads preloaded (HotArgs:
 // the activation code, the weights, the up matrix or group scales, the positions, offset terms or
 // grouped code's scales out, then the counts).
-template <int RTW, bool DUAL, int EPI, int NKC, bool ROPE, int KSW, bool GRP, int IN, int OUT, bool SEQ = false>
+template <int RTW, bool DUAL, int EPI, int NKC, bool ROPE, int KSW, bool GRP, int IN, int OUT, bool SEQ = false,
+          bool FIN = false>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(3)))
 gemm_skinny_hot_kernel(const void* p0, const void* p1, const void* p2, const void* p3, int tokens, int tt_count,
                        int rg_count, int splits, GemmArgs a) {
   constexpr int kKb = kernarg_bytes<const void*, const void*, const void*, const void*, int, int, int, int, GemmArgs>();
   gemm_skinny_body<RTW, DUAL, EPI, NKC, ROPE, KSW, false, kEpiStore, false, false, GRP, false, false, false, 16, kKb,
-                   IN, OUT, SEQ>(a, tt_count, rg_count, splits, a, 0, AttnMergeArgs{}, AttnFuseArgs{},
+                   IN, OUT, SEQ, FIN>(a, tt_count, rg_count, splits, a, 0, AttnMergeArgs{}, AttnFuseArgs{},
                             HotArgs{p0, p1, p2, p3, nullptr, nullptr, tokens});
 }
 
@@ -2563,21 +2626,52 @@ __device__ __forceinline__ float4 sum_splits4(const float* __restrict__ part, si
   return acc;
 }
 
+// The same for the pipelined GEMM's partials (int32 sums, or one split's finished fp32 sum): the exact sum
+// without its zero point 8 (256 sumH + sumL), rounded once.  |sum| < 2^33, so its double is exact.
+__device__ __forceinline__ float exact_sum(long long t) { return (float)(double)t; }
+__device__ __forceinline__ long long zero_point(int in_dim, int splits, int sum_h, int sum_l) {
+  return in_dim > kIntPartK * splits ? 0 : 8 * (256 * (long long)sum_h + (long long)sum_l);  // (ZOFF: off already)
+}
+__device__ __forceinline__ float4 exact_splits4(const float* __restrict__ part, size_t zstride, size_t off, int splits,
+                                                long long zero) {
+  if (splits == 1) return *reinterpret_cast<const float4*>(part + off);
+  long long t[4] = {-zero, -zero, -zero, -zero};
+  for (int z0 = 0; z0 < splits; z0 += 8) {
+    int4 pz[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      pz[u] = z0 + u < splits ? *reinterpret_cast<const int4*>(part + (size_t)(z0 + u) * zstride + off)
+                              : make_int4(0, 0, 0, 0);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      t[0] += pz[u].x;
+      t[1] += pz[u].y;
+      t[2] += pz[u].z;
+      t[3] += pz[u].w;
+    }
+  }
+  return make_float4(exact_sum(t[0]), exact_sum(t[1]), exact_sum(t[2]), exact_sum(t[3]));
+}
+
 // Sums the split partials in z order and applies the offset correction and the epilogue
 // (kEpiStore with bias, or kEpiResidual with bf16 rounding).  One thread per 4 outputs.
-template <int EPI>
+// EXACT (here and below): the pipelined GEMM's partials.
+template <int EPI, bool EXACT>
 __global__ void __launch_bounds__(256) gemm_splitk_reduce_kernel(GemmArgs a, int splits) {
   const size_t quads = (size_t)a.tokens * (a.out_dim / 4);
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= quads) return;
   const int tok = (int)(i / (a.out_dim / 4));
   const int row0 = (int)(i % (a.out_dim / 4)) * 4;
-  const float4 acc = sum_splits4(a.part, (size_t)a.tokens * a.out_dim, (size_t)tok * a.out_dim + row0, splits);
+  const size_t zstride = (size_t)a.tokens * a.out_dim, off = (size_t)tok * a.out_dim + row0;
+  const float4 acc = EXACT ? exact_splits4(a.part, zstride, off, splits,
+                                           zero_point(a.in_dim, splits, a.sums[2 * tok], a.sums[2 * tok + 1]))
+                           : sum_splits4(a.part, zstride, off, splits);
   const double corr = -8.0 * (256.0 * (double)a.sums[2 * tok] + (double)a.sums[2 * tok + 1]) * (double)a.sx[tok];
   float out[4] = {acc.x, acc.y, acc.z, acc.w};
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const float v = out[q] + (float)(corr * (double)a.sw[row0 + q]);
+    const float v = EXACT ? out[q] * a.sx[tok] * a.sw[row0 + q] : out[q] + (float)(corr * (double)a.sw[row0 + q]);
     if (EPI == kEpiResidual) {
       const float o = a.resid[(size_t)tok * a.resid_stride + row0 + q] + v;
       out[q] = a.round_bf16 ? round_bf16(o) : o;
@@ -2592,7 +2686,7 @@ __global__ void __launch_bounds__(256) gemm_splitk_reduce_kernel(GemmArgs a, int
 // kEpiResidual: residual, optional raw copy, optional bf16 rounding), the finished row written to
 // a.y, then RMSNorm(norm_w) + two-limb quantization of that row into xq_out / sx_out / sums_out.
 // Thread t owns float4 columns t and t + 256.  grid = tokens, block = 256.
-template <int EPI>
+template <int EPI, bool EXACT>
 __global__ void __launch_bounds__(256) reduce_norm_quant_kernel(GemmArgs a, int splits) {
   const int tok = blockIdx.x;
   const int n4 = a.out_dim >> 2;
@@ -2604,11 +2698,14 @@ __global__ void __launch_bounds__(256) reduce_norm_quant_kernel(GemmArgs a, int 
     v[j] = make_float4(0, 0, 0, 0);
     if (k >= n4) continue;
     const int row0 = 4 * k;
-    const float4 acc = sum_splits4(a.part, (size_t)a.tokens * a.out_dim, (size_t)tok * a.out_dim + row0, splits);
+    const size_t zstride = (size_t)a.tokens * a.out_dim, off = (size_t)tok * a.out_dim + row0;
+    const float4 acc = EXACT ? exact_splits4(a.part, zstride, off, splits,
+                                             zero_point(a.in_dim, splits, a.sums[2 * tok], a.sums[2 * tok + 1]))
+                             : sum_splits4(a.part, zstride, off, splits);
     float out[4] = {acc.x, acc.y, acc.z, acc.w};
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const float val = out[q] + (float)(corr * (double)a.sw[row0 + q]);
+      const float val = EXACT ? out[q] * a.sx[tok] * a.sw[row0 + q] : out[q] + (float)(corr * (double)a.sw[row0 + q]);
       if (EPI == kEpiResidual) {
         out[q] = a.resid[(size_t)tok * a.resid_stride + row0 + q] + val;
       } else {
@@ -2640,7 +2737,7 @@ __global__ void __launch_bounds__(256) reduce_norm_quant_kernel(GemmArgs a, int 
 // bias or a stand-in, p2 row scales, p3 norm weights or a stand-in, p4 limb sums, p5 scales, n0 the
 // token count), the flags read from `a` after the loads are issued; the outputs are the token's row
 // of a.xq_out (chunk_stride 256), a.sx_out and a.sums_out, whatever xq_row, sx_out and sums_out say.
-template <int EPI, int ZB, class Issue, int W, bool HOT>
+template <int EPI, int ZB, class Issue, int W, bool HOT, int EXACT>
 __device__ __forceinline__ void reduce_norm_quant_row_zb(const GemmArgs& a, int splits, int tok, int8_t* xq_row,
                                                          int chunk_stride, float* sx_out, int* sums_out, bool write_y,
                                                          Issue&& issue, const HotArgs& hot) {
@@ -2679,16 +2776,53 @@ __device__ __forceinline__ void reduce_norm_quant_row_zb(const GemmArgs& a, int 
     ad[j] = r4[LS * j];
     wn[j] = w4[LS * j];
   }
-  // split sums in z order
+  // split sums in z order (EXACT: in integers, of groups whose sum fits int32, kExactNarrow: of all; one split,
+  // ZB = 1, holds the finished sum)
+  constexpr bool kInt = EXACT != 0 && ZB > 1, kWide = EXACT == kExactWide;
+  constexpr int kGroup = kWide ? (HOT ? 2 : 3) : ZB;
+  long long tot[kInt ? NV : 1][4];
 #pragma unroll
   for (int j = 0; j < NV; ++j) acc[j] = make_float4(0, 0, 0, 0);
+#pragma unroll
+  for (int j = 0; j < (kInt ? NV : 1); ++j) tot[j][0] = tot[j][1] = tot[j][2] = tot[j][3] = 0;
+  float4 pz[ZB][NV];
+  auto add_exact = [&](int z0) {
+    if (!kWide || z0 + ZB <= splits) {
+#pragma unroll
+      for (int u0 = 0; u0 < ZB; u0 += kGroup)
+#pragma unroll
+        for (int j = 0; j < (kInt ? NV : 1); ++j) {
+          uint32_t t[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+          for (int u = u0; u < (u0 + kGroup < ZB ? u0 + kGroup : ZB); ++u) {
+            const bool live = kWide || z0 + u < splits;
+            t[0] += live ? __float_as_uint(pz[u][j].x) : 0u;
+            t[1] += live ? __float_as_uint(pz[u][j].y) : 0u;
+            t[2] += live ? __float_as_uint(pz[u][j].z) : 0u;
+            t[3] += live ? __float_as_uint(pz[u][j].w) : 0u;
+          }
+#pragma unroll
+          for (int q = 0; q < 4; ++q) tot[j][q] = kWide ? tot[j][q] + (int)t[q] : (int)((uint32_t)tot[j][q] + t[q]);
+        }
+    } else {  // fewer splits: one by one
+#pragma unroll
+      for (int u = 0; u < ZB; ++u)
+        if (z0 + u < splits)
+#pragma unroll
+          for (int j = 0; j < (kInt ? NV : 1); ++j) {
+            tot[j][0] += __float_as_int(pz[u][j].x);
+            tot[j][1] += __float_as_int(pz[u][j].y);
+            tot[j][2] += __float_as_int(pz[u][j].z);
+            tot[j][3] += __float_as_int(pz[u][j].w);
+          }
+    }
+  };
   if constexpr (HOT) {
     // splits <= ZB (the launcher checks), straight-line: every split's loads issued unconditionally
     // (past the last split the last again, unused; without splits the row scales), `issue`, then the
     // adds as selects (adding +0 leaves a sum that started at +0 unchanged)
     const float4* pt0 = splits > 0 ? pt : sw4;
     const int zlast = max(splits, 1) - 1;
-    float4 pz[ZB][NV];
 #pragma unroll
     for (int u = 0; u < ZB; ++u)
 #pragma unroll
@@ -2700,20 +2834,23 @@ __device__ __forceinline__ void reduce_norm_quant_row_zb(const GemmArgs& a, int 
     xq_row = a.xq_out + (size_t)tok * (2 * QWEN_HIDDEN);
     sx_out = a.sx_out + tok;
     sums_out = a.sums_out + 2 * tok;
+    if constexpr (kInt) {
+      add_exact(0);
+    } else {
 #pragma unroll
-    for (int u = 0; u < ZB; ++u) {
-      const bool live = u < splits;
+      for (int u = 0; u < ZB; ++u) {
+        const bool live = u < splits;
 #pragma unroll
-      for (int j = 0; j < NV; ++j) {
-        acc[j].x += live ? pz[u][j].x : 0.0f;
-        acc[j].y += live ? pz[u][j].y : 0.0f;
-        acc[j].z += live ? pz[u][j].z : 0.0f;
-        acc[j].w += live ? pz[u][j].w : 0.0f;
+        for (int j = 0; j < NV; ++j) {
+          acc[j].x += live ? pz[u][j].x : 0.0f;
+          acc[j].y += live ? pz[u][j].y : 0.0f;
+          acc[j].z += live ? pz[u][j].z : 0.0f;
+          acc[j].w += live ? pz[u][j].w : 0.0f;
+        }
       }
     }
   }
   for (int z0 = 0; !HOT && z0 < splits; z0 += ZB) {
-    float4 pz[ZB][NV];
 #pragma unroll
     for (int u = 0; u < ZB; ++u)
 #pragma unroll
@@ -2723,16 +2860,20 @@ __device__ __forceinline__ void reduce_norm_quant_row_zb(const GemmArgs& a, int 
       issue();
       __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (kInt) {
+      add_exact(z0);
+    } else {
 #pragma unroll
-    for (int u = 0; u < ZB; ++u)
-      if (z0 + u < splits)
+      for (int u = 0; u < ZB; ++u)
+        if (z0 + u < splits)
 #pragma unroll
-        for (int j = 0; j < NV; ++j) {
-          acc[j].x += pz[u][j].x;
-          acc[j].y += pz[u][j].y;
-          acc[j].z += pz[u][j].z;
-          acc[j].w += pz[u][j].w;
-        }
+          for (int j = 0; j < NV; ++j) {
+            acc[j].x += pz[u][j].x;
+            acc[j].y += pz[u][j].y;
+            acc[j].z += pz[u][j].z;
+            acc[j].w += pz[u][j].w;
+          }
+    }
   }
   if (!HOT && splits < 1) issue();  // the caller's loads are issued exactly once, also without splits
   const bool has_add = EPI == kEpiResidual || a.bias != nullptr;
@@ -2742,11 +2883,19 @@ __device__ __forceinline__ void reduce_norm_quant_row_zb(const GemmArgs& a, int 
     if (!has_add) ad[j] = make_float4(0, 0, 0, 0);
     if (!has_w) wn[j] = make_float4(0, 0, 0, 0);
   }
-  const double corr = -8.0 * (256.0 * (double)sum_h + (double)sum_l) * (double)sx_tok;
+  if constexpr (kInt) {
+    const long long zero = zero_point(a.in_dim, splits, sum_h, sum_l);
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+      acc[j] = make_float4(exact_sum(tot[j][0] - zero), exact_sum(tot[j][1] - zero), exact_sum(tot[j][2] - zero),
+                           exact_sum(tot[j][3] - zero));
+  }
+  const double corr =
+      EXACT ? (double)sx_tok : -8.0 * (256.0 * (double)sum_h + (double)sum_l) * (double)sx_tok;
   float4 v[NV];
 #pragma unroll
   for (int j = 0; j < NV; ++j)
-    v[j] = rnq_combine<EPI>(a, tok, 4 * (lane + LS * j), acc[j], sw[j], ad[j], corr, write_y);
+    v[j] = rnq_combine<EPI, EXACT != 0>(a, tok, 4 * (lane + LS * j), acc[j], sw[j], ad[j], corr, write_y);
   // RMSNorm (norm_quant_row's arithmetic, wave reductions)
   if (a.norm == kNormDecode) {
     double ss = 0.0;
@@ -2986,22 +3135,22 @@ __device__ __forceinline__ void reduce_norm_quant_row(const GemmArgs& a, int spl
 // grid = tokens, block = 128 (two waves per row: half the per-lane work of the one-wave form, three
 // LDS exchanges); the values equal the one-wave form's except the norm's sum of squares, added in
 // another order.
-template <int EPI>
+template <int EPI, int EXACT>
 __global__ void __launch_bounds__(128) reduce_norm_quant_pair_kernel(GemmArgs a, int splits) {
   touch_kernargs<kernarg_bytes<GemmArgs, int>()>();
   const int tok = blockIdx.x;
   int8_t* xq_row = a.xq_out + (size_t)tok * (2 * QWEN_HIDDEN);
   if (splits == 1)
-    reduce_norm_quant_row_zb<EPI, 1, NoIssue, 2>(a, splits, tok, xq_row, 256, a.sx_out + tok, a.sums_out + 2 * tok, true,
-                                                  NoIssue{});
+    reduce_norm_quant_row_zb<EPI, 1, NoIssue, 2, false, EXACT>(a, splits, tok, xq_row, 256, a.sx_out + tok,
+                                                               a.sums_out + 2 * tok, true, NoIssue{});
   else
-    reduce_norm_quant_row_zb<EPI, 5, NoIssue, 2>(a, splits, tok, xq_row, 256, a.sx_out + tok, a.sums_out + 2 * tok, true,
-                                                  NoIssue{});
+    reduce_norm_quant_row_zb<EPI, EXACT != 0 ? 7 : 5, NoIssue, 2, false, EXACT>(a, splits, tok, xq_row, 256, a.sx_out + tok,
+                                                               a.sums_out + 2 * tok, true, NoIssue{});
 }
 
 // The same with the first loads' operands preloaded (HotArgs of reduce_norm_quant_row_zb), residual
 // rows 1536 floats apart.
-template <int EPI>
+template <int EPI, int EXACT>
 __global__ void __launch_bounds__(128) reduce_norm_quant_pair_hot_kernel(const void* p0, const void* p1, const void* p2,
                                                                          const void* p3, const void* p4, const void* p5,
                                                                          int tokens, int splits, GemmArgs a) {
@@ -3012,11 +3161,11 @@ __global__ void __launch_bounds__(128) reduce_norm_quant_pair_hot_kernel(const v
   const int tok = blockIdx.x;
   // (the outputs are addressed inside, once the loads are issued)
   if (splits == 1)
-    reduce_norm_quant_row_zb<EPI, 1, decltype(issue)&, 2, true>(a, splits, tok, nullptr, 256, nullptr, nullptr, true,
-                                                                issue, hot);
+    reduce_norm_quant_row_zb<EPI, 1, decltype(issue)&, 2, true, EXACT>(a, splits, tok, nullptr, 256, nullptr, nullptr,
+                                                                       true, issue, hot);
   else
-    reduce_norm_quant_row_zb<EPI, 5, decltype(issue)&, 2, true>(a, splits, tok, nullptr, 256, nullptr, nullptr, true,
-                                                                issue, hot);
+    reduce_norm_quant_row_zb<EPI, 5, decltype(issue)&, 2, true, EXACT>(a, splits, tok, nullptr, 256, nullptr, nullptr,
+                                                                       true, issue, hot);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -3737,24 +3886,35 @@ static void launch_gemm_t(const GemmArgs& a, hipStream_t st) {
   hipLaunchKernelGGL((gemm_i8_kernel<NT, KSPLIT, EPI, DUAL>), grid, dim3(256), 0, st, a);
 }
 
-// The reduce step after a GEMM that wrote fp32 partials: plain (bias / residual epilogue) or fused.
-template <int EPI>
+// The reduce step after a GEMM that wrote partials (EXACT: the pipelined GEMM's): plain (bias / residual
+// epilogue) or fused.
+template <int EPI, bool EXACT = false>
 static void launch_reduce(const GemmArgs& a, int splits, hipStream_t st) {
   if (a.fuse == kFuseNormQuant) {
-    if (a.out_dim == QWEN_HIDDEN && splits <= 5 && (EPI != kEpiResidual || a.resid_stride == QWEN_HIDDEN)) {
-      // the first loads' operands preloaded (an absent bias or norm weight read from the row scales)
-      const void* add = EPI == kEpiResidual ? (const void*)a.resid : a.bias ? (const void*)a.bias : a.sw;
-      const void* nw = a.norm != kNormNone ? (const void*)a.norm_w : a.sw;
-      hipLaunchKernelGGL((reduce_norm_quant_pair_hot_kernel<EPI>), dim3(a.tokens), dim3(128), 0, st,
-                         (const void*)a.part, add, (const void*)a.sw, nw, (const void*)a.sums, (const void*)a.sx,
-                         a.tokens, splits, a);
-    } else if (a.out_dim == QWEN_HIDDEN)
-      hipLaunchKernelGGL((reduce_norm_quant_pair_kernel<EPI>), dim3(a.tokens), dim3(128), 0, st, a, splits);
+    auto go = [&](auto form) {
+      constexpr int kForm = decltype(form)::value;
+      if (a.out_dim == QWEN_HIDDEN && splits <= 5 && (EPI != kEpiResidual || a.resid_stride == QWEN_HIDDEN)) {
+        // the first loads' operands preloaded (an absent bias or norm weight read from the row scales)
+        const void* add = EPI == kEpiResidual ? (const void*)a.resid : a.bias ? (const void*)a.bias : a.sw;
+        const void* nw = a.norm != kNormNone ? (const void*)a.norm_w : a.sw;
+        hipLaunchKernelGGL((reduce_norm_quant_pair_hot_kernel<EPI, kForm>), dim3(a.tokens), dim3(128), 0, st,
+                           (const void*)a.part, add, (const void*)a.sw, nw, (const void*)a.sums, (const void*)a.sx,
+                           a.tokens, splits, a);
+      } else if (a.out_dim == QWEN_HIDDEN) {
+        hipLaunchKernelGGL((reduce_norm_quant_pair_kernel<EPI, kForm>), dim3(a.tokens), dim3(128), 0, st, a, splits);
+      } else {
+        hipLaunchKernelGGL((reduce_norm_quant_kernel<EPI, EXACT>), dim3(a.tokens), dim3(256), 0, st, a, splits);
+      }
+    };
+    if (!EXACT)
+      go(std::integral_constant<int, 0>{});
+    else if (a.in_dim <= kIntPartK)
+      go(std::integral_constant<int, EXACT ? kExactNarrow : 0>{});
     else
-      hipLaunchKernelGGL((reduce_norm_quant_kernel<EPI>), dim3(a.tokens), dim3(256), 0, st, a, splits);
+      go(std::integral_constant<int, EXACT ? kExactWide : 0>{});
   } else {
     const size_t quads = (size_t)a.tokens * (a.out_dim / 4);
-    hipLaunchKernelGGL((gemm_splitk_reduce_kernel<EPI>), dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, a,
+    hipLaunchKernelGGL((gemm_splitk_reduce_kernel<EPI, EXACT>), dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, a,
                        splits);
   }
 }
@@ -3771,6 +3931,14 @@ static void launch_gemm_pipe_t(const GemmArgs& a, int splits, hipStream_t st) {
     hipLaunchKernelGGL((gemm_i8_pipe_kernel<NT, RTW, NBUF, EPI, DUAL, TW, WPE, OWN, ROPE, decltype(ef)::value, BATCH>),
                        grid, dim3(256 * TW), 0, st, a);
   };
+  if constexpr (!DUAL && !ROPE) {
+    if (splits > 1 && a.in_dim > kIntPartK * splits) {
+      hipLaunchKernelGGL((gemm_i8_pipe_kernel<NT, RTW, NBUF, EPI, DUAL, TW, WPE, OWN, ROPE, 0, BATCH, true>), grid,
+                         dim3(256 * TW), 0, st, a);
+      launch_reduce<EPI, true>(a, splits, st);
+      return;
+    }
+  }
   if constexpr (EPI == kEpiSiluMul) {
     if (a.prefill_silu)
       int_sum ? go(std::integral_constant<int, kEfPrefillSilu | kEfIntSum>{})
@@ -3784,13 +3952,14 @@ static void launch_gemm_pipe_t(const GemmArgs& a, int splits, hipStream_t st) {
   }
   // K splits, or an epilogue fused into the reduce step, finish in the reduce kernel; the prefill RoPE
   // epilogue is complete in the GEMM itself
-  if (!DUAL && !ROPE && (splits > 1 || a.fuse != kFuseNone)) launch_reduce<EPI>(a, splits, st);
+  if (!DUAL && !ROPE && (splits > 1 || a.fuse != kFuseNone)) launch_reduce<EPI, true>(a, splits, st);
 }
 
 // Skinny GEMMs for at most kSkinnyTokens tokens with in_dim 1536 (12 K chunks in one block) or 8960
 // (5 splits of 14 chunks, finished by the reduce step).  Returns false for other shapes.
 
-template <int RTW, bool DUAL, int EPI, int NKC, bool ROPE, int KSW = 1, bool GRP = false, bool SEQ = false>
+template <int RTW, bool DUAL, int EPI, int NKC, bool ROPE, int KSW = 1, bool GRP = false, bool SEQ = false,
+          bool FIN = false>
 static void launch_skinny_t(const GemmArgs& a, int rg_count, int splits, hipStream_t st) {
   // the grouped code's per-group sums are only finished by the split-K partial epilogue
   if (GRP && splits <= 1) throw std::runtime_error("grouped-code GEMM needs the split-K partial epilogue");
@@ -3803,13 +3972,13 @@ static void launch_skinny_t(const GemmArgs& a, int rg_count, int splits, hipStre
   if (kIn > 0 && a.in_dim == kIn && a.out_dim == kOut && splits * NKC * kKChunk == kIn) {
     const void* p2 = GRP ? (const void*)a.gsx : DUAL ? (const void*)a.wp2 : nullptr;
     const void* p3 = GRP ? (const void*)a.gcorr : ROPE ? (const void*)a.pos : DUAL ? (const void*)a.gsx_out : nullptr;
-    hipLaunchKernelGGL((gemm_skinny_hot_kernel<RTW, DUAL, EPI, NKC, ROPE, KSW, GRP, kIn, kOut, SEQ>), dim3(blocks),
+    hipLaunchKernelGGL((gemm_skinny_hot_kernel<RTW, DUAL, EPI, NKC, ROPE, KSW, GRP, kIn, kOut, SEQ, FIN>), dim3(blocks),
                        dim3(256 * KSW), 0, st, (const void*)a.xq, (const void*)a.wp, p2, p3, a.tokens, tt, rg_count,
                        splits, a);
     return;
   }
-  if constexpr (SEQ) {
-    throw std::runtime_error("prefill RoPE epilogue: the [q | k | v] projection only");
+  if constexpr (SEQ || FIN) {
+    throw std::runtime_error("prefill epilogues: the [q | k | v] and O projections only");
   } else {
     hipLaunchKernelGGL((gemm_skinny_kernel<RTW, DUAL, EPI, NKC, ROPE, KSW, GRP>), dim3(blocks), dim3(256 * KSW), 0, st,
                        a, tt, rg_count, splits);
@@ -3844,6 +4013,18 @@ static bool launch_skinny(const GemmArgs& a, hipStream_t st) {
       return true;
     }
     if (!DUAL && a.fuse != kFuseNone && !a.part) return false;
+    if constexpr (!DUAL && EPI == kEpiStore) {
+      if (a.fuse == kFuseNormQuant && a.zero_sums && a.out_dim == QWEN_HIDDEN) {  // finished partials
+        if (a.tokens > 16)
+          launch_skinny_t<1, false, EPI, 12, false, 2, false, false, true>(a, row_tiles / 4, 1, st);
+        else
+          launch_skinny_t<1, false, EPI, 12, false, 1, false, false, true>(a, row_tiles / 4, 1, st);
+        GemmArgs r = a;
+        r.sums = a.zero_sums;
+        launch_reduce<EPI>(r, 1, st);
+        return true;
+      }
+    }
     // the O shape over more than one token tile: two wave groups split K, as Q/K/V (64 x 4096 decode
     // +0.25%, interleaved; the sums are exact int32, so the bits are the same)
     if (!DUAL && a.tokens > 16 && a.out_dim == QWEN_HIDDEN)
