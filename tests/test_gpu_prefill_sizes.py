@@ -37,7 +37,8 @@ def run(model, mode, x, batch, seq, past, seed, layers):
 
 @pytest.mark.parametrize("batch,seq,past", [(1, 65, 0), (1, 130, 0), (3, 90, 0), (1, 257, 0), (1, 400, 0), (2, 400, 33),
                                             (1, 1025, 0), (1, 5, 3000), (1, 16, 700), (1, 33, 2047), (2, 70, 1500),
-                                            (1, 1, 0), (1, 17, 0), (3, 21, 5), (64, 1, 7), (1, 64, 0)])
+                                            (1, 1, 0), (1, 17, 0), (3, 21, 5), (64, 1, 7), (1, 64, 0),
+                                            (1, 2100, 0), (2, 1500, 0), (3, 1661, 0)])
 def test_layer_against_ordered(model, batch, seq, past):
     import torch
 

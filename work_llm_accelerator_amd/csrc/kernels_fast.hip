@@ -4048,6 +4048,18 @@ static bool launch_skinny(const GemmArgs& a, hipStream_t st) {
   return false;
 }
 
+// CUs of the current device.
+static int device_cus() {
+  static const int cus = [] {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1)
+      return 256;
+    return n;
+  }();
+  return cus;
+}
+
 // K splits of the two-blocks-per-CU pipelined GEMM with blocks of `tok` tokens and `tiles` row tiles: the least
 // of the time of its rounds (`alone` us per K chunk of a block alone on its CU, `pair` of two) and of the
 // partials' write and read, 2 us for the reduce launch where the call has none anyway.
@@ -4351,27 +4363,58 @@ size_t attn_prefill_workspace_bytes(int keys, int nseq) {
 }
 
 AttnPrefillPlan plan_attn_prefill(int S, int past, int nseq) {
+  // Times in key tiles of a block alone on its CU (1.2 us).  A block takes its tiles and kEnds for its start and
+  // end; of two blocks on a CU each takes kPair times as long, and the CUs together no less than kShare times
+  // their even share.  Splits add the merge (about 2 to the quantization it replaces) and kPartial per block for
+  // the partials' write and read.
+  // Without splits and with more blocks than CUs, the blocks that share a CU from the start (j and j + CUs in
+  // dispatch order: the query tiles of a sequence and KV head, longest first) differ in length, so the longer
+  // one runs alone at the end.
+  // Fitted to layers of 1 to 8 sequences of 64 to 4096 tokens with histories of up to 12000 keys, unsplit and
+  // with up to 64 splits (medians of interleaved runs): the plan's layer is at most 1.3% slower than the unsplit
+  // one.  2 x 2600 tokens 629 us unsplit, 659 with two splits; 3 x 1661 560 and 574; 5 x 784 429 and 439;
+  // 1 x 4096 623 and 575; 1 x 2100 338 and, with four, 321.
+  constexpr double kEnds = 4.0, kPair = 2.0, kShare = 1.1, kMerge = 2.0, kPartial = 0.03;
+  constexpr double kMargin = 0.95;  // more blocks than CUs: the gain that a split has to promise
+  const int cus = device_cus();
   const int ntiles = (past + S + kPfKeys - 1) / kPfKeys;
   const int qtiles = (S + kPfQ - 1) / kPfQ;
-  AttnPrefillPlan best{1, ntiles};
-  double cost = 0.0;
-  // The time in tiles of a block alone on its CU (1.2 us): its tiles and about 4 for its start and end while
-  // every block has a CU; two blocks on a CU take 2.2 times as long per tile, and the CUs share what there
-  // is.  The partials' write and read add 100 KB per block, the merge about 2 to the quantization it replaces.
-  for (int n = 1; n <= kAttnMaxSplits && n <= ntiles; ++n) {
-    const int tps = (ntiles + n - 1) / n;
-    if (n > 1 && tps == (ntiles + n - 2) / (n - 1)) continue;  // same tiles per split: fewer splits
-    double total = 0.0, blocks = 0.0;
-    for (int q = 0; q < qtiles; ++q) {
-      const int last = past + (q * kPfQ + kPfQ < S ? q * kPfQ + kPfQ : S) - 1;
-      total += last / kPfKeys + 1;
-      blocks += last / kPfKeys / tps + 1;
+  const long long rows = (long long)QWEN_KV_HEADS * nseq;
+  // query tiles that reach key tile x
+  auto reach = [&](int x) -> long long {
+    const long long before = (long long)x * kPfKeys - past;  // queries whose keys end before it
+    return before <= 0 ? qtiles : S <= before ? 0 : qtiles - before / kPfQ;
+  };
+  double total = 0.0;  // key tiles of all blocks
+  for (int x = 0; x < ntiles; ++x) total += (double)reach(x);
+  total *= (double)rows;
+  auto share = [&](double blocks) { return kShare * (total + kEnds * blocks) / cus; };
+  const double blocks1 = (double)(rows * qtiles);
+  double cost1 = ntiles + kEnds;
+  if (blocks1 > cus) {
+    auto length = [&](long long b) {
+      const int q = qtiles - 1 - (int)(b % qtiles);
+      return (past + (q * kPfQ + kPfQ < S ? q * kPfQ + kPfQ : S) - 1) / kPfKeys + 1 + kEnds;
+    };
+    cost1 = share(blocks1);
+    for (long long b = 0; b < cus; ++b) {
+      const double x = length(b), y = b + cus < rows * qtiles ? length(b + cus) : 0.0;
+      const double pair = x < y ? kPair * x + (y - x) : kPair * y + (x - y);
+      if (pair > cost1) cost1 = pair;
     }
-    total *= 2.0 * nseq;
-    blocks *= 2.0 * nseq;
-    const double alone = tps + 4.0, share = 1.1 * (total + 4.0 * blocks) / 256.0;
-    const double c = (blocks <= 256.0 ? alone : share > 2.2 * alone ? share : 2.2 * alone) + (n > 1 ? 2.0 + blocks * 0.03 : 0.0);
-    if (n == 1 || c < cost) {
+  }
+  AttnPrefillPlan best{1, ntiles};
+  double cost = blocks1 > cus ? kMargin * cost1 : cost1;
+  if (blocks1 > cus && cost <= share(blocks1) + kMerge) return best;  // no split can gain
+  for (int n = 2; n <= kAttnMaxSplits && n <= ntiles; ++n) {
+    const int tps = (ntiles + n - 1) / n;
+    if (tps == (ntiles + n - 2) / (n - 1)) continue;  // same tiles per split: fewer splits
+    double blocks = 0.0;
+    for (int x = 0; x < ntiles; x += tps) blocks += (double)reach(x);
+    blocks *= (double)rows;
+    const double alone = tps + kEnds, even = share(blocks);
+    const double c = (blocks <= cus ? alone : even > kPair * alone ? even : kPair * alone) + kMerge + kPartial * blocks;
+    if (c < cost) {
       cost = c;
       best = AttnPrefillPlan{n, tps};
     }
