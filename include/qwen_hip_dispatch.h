@@ -54,7 +54,7 @@ int qwen_hip_prefill_dispatch_layers(const qwen_prefill_descriptor* descriptors,
  * codes, completed count and results (bit for bit) as qwen_hip_decode_dispatch_layers, except that it
  * calls no allocating routine (no hipMalloc / hipFree, no allocating library call) and does not
  * synchronize: every layer is queued on `stream` and the call returns.  The intermediates of the layer
- * being run live in one static device array of 147,456 bytes per GPU (one token's workspace, the
+ * being run live in one static device array of 69,376 bytes per GPU (one token's workspace, the
  * attention output row, the descriptor's RoPE row and position), held until the process ends; one
  * token per descriptor fixes that need, so no argument can exceed it.  The array keeps the last
  * call's contents, and every value a layer reads from it is written earlier in the same call.  Calls

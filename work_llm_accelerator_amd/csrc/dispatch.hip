@@ -26,12 +26,12 @@ using namespace qwen;
 // process ends; host code reaches it only through the address hipGetSymbolAddress returns for the
 // current device (the array's name is a host-side stand-in, not a device address).
 // ---------------------------------------------------------------------------------------------
-constexpr size_t kNoAllocWorkspaceFloats = 35072;  // decode_workspace_floats(1)
+constexpr size_t kNoAllocWorkspaceFloats = decode_workspace_floats(1);
 constexpr size_t kNoAllocAttOffset = kNoAllocWorkspaceFloats;             // attention output row
 constexpr size_t kNoAllocRopeOffset = kNoAllocAttOffset + QWEN_HIDDEN;    // cos[64] | sin[64]
 constexpr size_t kNoAllocPosOffset = kNoAllocRopeOffset + QWEN_HEAD_DIM;  // the position (an int)
-constexpr size_t kNoAllocScratchFloats = 36864;                          // 147,456 bytes in all
-static_assert(kNoAllocPosOffset < kNoAllocScratchFloats, "scratch layout");
+constexpr size_t kNoAllocScratchFloats = kNoAllocPosOffset + 64;
+static_assert(kNoAllocScratchFloats * sizeof(float) == 69376, "the size that qwen_hip_dispatch.h states");
 static __device__ __align__(256) float scratch[kNoAllocScratchFloats];
 
 namespace {
@@ -185,8 +185,6 @@ int qwen_hip_decode_dispatch_layers_noalloc(const qwen_decode_descriptor* dsc, i
   set_completed(completed, 0);
   if (!dsc || n <= 0) return QWEN_ERR_DECODE_DESC;  // qwen_decode_top_wrapper.cpp:118-120
   return guarded_dispatch([&]() -> int {
-    if (decode_workspace_floats(1) > kNoAllocWorkspaceFloats)
-      throw std::runtime_error("one token's decode workspace exceeds the static scratch");
     const hipStream_t st = static_cast<hipStream_t>(stream);
     float* base = noalloc_scratch();
     const DecodeWorkspace w = carve_decode_workspace(base, 1);

@@ -39,8 +39,7 @@ void launch_rope_prefill(float* q, float* k_rows, const float* rope, int tokens,
 void launch_rope_table_prefill(float* rope, int first, int count, hipStream_t st);
 // prefill: token b is the query at position past + b over keys 0..past+b of one sequence's rows.
 void launch_attention_ordered(const float* q, const float* k_cache, const float* v_cache, size_t cache_stride,
-                              const int* pos, int max_keys, int tokens, bool prefill, int past, float* ctx,
-                              hipStream_t st);
+                              const int* pos, int max_keys, int tokens, float* ctx, hipStream_t st);
 
 // The same attention with the scores of every key kept in `scores` (attention_ordered_scores floats)
 // between its two launches.  k_new / v_new given (decode, one token): q and the new key are rotated with

@@ -117,8 +117,8 @@ __device__ __forceinline__ double chain_add(double acc, const double* v) {
 // RMSNorm.  decode: double serial sum (qwen_decode_attention_kernel.cpp:13-27);
 // prefill: float serial sum + approx_sqrt (qwen_prefill_attention_kernel.cpp:112-126).
 // All threads form the squares (the square of a float is exact in double, so adding the finished
-// square is the reference's step); wave 0 adds them in order.  Bound by the 1536-step chain: 6.8 us
-// (18.2 us when one thread also loaded and multiplied), 6.7 us for the prefill form of 128 rows (15.2).
+// square is the reference's step); wave 0 adds them in order.  Bound by the 1536-step chain: 8.9 us
+// for 7 decode rows (20.5 us when one thread also loaded and multiplied), 8.9 us for 128 prefill rows (15.3).
 // grid.x = tokens, block = 256.
 // ---------------------------------------------------------------------------------------------
 struct RmsScratch {
@@ -235,12 +235,12 @@ __device__ __forceinline__ OrdSegment pick_segment(const OrdProject& a, int row)
 // prefetched PD chunks ahead in registers, the input row in LDS).  A ring of three product chunks: at
 // barrier c the chunks up to c + 1 are finished, so the adding waves read ahead across the chunk
 // boundary while chunk c + 2 is formed.
-// R = 16: 96 to 128 blocks; the gate/up pair takes R = 64 (32 rows of each matrix, so that SiLU * up
+// R = 16: 96 to 128 blocks, 1120 for the gate/up pair (8 rows of each matrix a block, so that SiLU * up
 // needs no further launch).  NORM: the input row is RMS-normalized (decode) by every block, a 1536-step
 // f64 chain that a launch of its own would also take, plus the launch.
-// One token, before (one thread per output row that also unpacked, scaled and multiplied; 6 blocks for 1536
-// rows) and now: q/k/v with the norm 123 -> 11 us (three launches and the norm's before), o 36 -> 6.7 us,
-// gate/up with the norm 93 -> 19 us, down (8960 steps) 196 -> 27.6 us.
+// One token, traced in a resident decode step, before (one thread per output row that also unpacked, scaled and
+// multiplied; 6 blocks for 1536 rows) and now: q/k/v with the norm 121 -> 13.1 us (three launches and the norm's
+// before), o 36 -> 7.8 us, gate/up with the norm 93 -> 20.2 us, down (8960 steps) 196 -> 31.4 us.
 template <int R, int KC, int PD, int K, bool NORM, bool GU>
 __global__ void __launch_bounds__(256 + 4 * R) project_chain_kernel(OrdProject a) {
   constexpr int kAdders = 4 * R;             // threads of the adding waves
@@ -372,8 +372,8 @@ __global__ void __launch_bounds__(256 + 4 * R) project_chain_kernel(OrdProject a
 // of one block per CU, where it would stand in the way of the only wave on each SIMD.  TT = 1, 2, 4, 8 (4x4x1) or 16 (16x16x1): launch_mfma.
 // The products cost the SIMD 2 cycles per token and input for 64 rows beside the add's 4 (a matrix
 // instruction of 8 cycles makes 4 tokens' products; it does not overlap the VALU), against 4 + 4 and the
-// weight's unpacking on the VALU.  One layer of 128 tokens: q/k/v 414 -> 25 us, o 138 -> 25, gate/up
-// 320 -> 150, down about 700 -> 131 us.
+// weight's unpacking on the VALU.  One layer of 128 tokens, traced: q/k/v 405 -> 26 us, o 138 -> 26, gate/up
+// 319 -> 152, down 784 -> 128 us.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kMmRows = 64;
@@ -544,7 +544,7 @@ project_mfma_kernel(OrdProject a) {
           schedule_fence();
         }
       });
-      if (c + PD < nc) load_x(c + PD, d);  
+      if (c + PD < nc) load_x(c + PD, d);
       // LDS operations of a wave finish in order: all but the last reads ahead are done, this wave's writes of
       // chunk c + 2 among them
       asm volatile("s_waitcnt lgkmcnt(%0)\n\ts_barrier" ::"n"(kAhead) : "memory");
@@ -668,23 +668,21 @@ __global__ void rope_table_prefill_kernel(float* __restrict__ rope, int first, i
 }
 
 // ---------------------------------------------------------------------------------------------
-// Two-pass softmax attention, one block of 128 threads per (head, query token).
-// decode: decode_attention_context (qwen_decode_attention_kernel.cpp:113-162), keys 0..pos[b],
-//         scaling (float)(1/sqrt(128)), host-compatible expf;
-// prefill: prefill_attention_context_block (qwen_prefill_attention_kernel.cpp:204-289), keys
-//         0..t, scaling 0.08838834764831845f, approx_exp.
+// Two-pass softmax attention of decode tokens, one block of 128 threads per (head, token): the form without
+// memory for the scores (the allocation-free dispatch).  decode_attention_context
+// (qwen_decode_attention_kernel.cpp:113-162), keys 0..pos[b], scaling (float)(1/sqrt(128)), host-compatible expf.
 // Pass 1 takes the max with the reference's `new > old` rule (any order gives the same value).
 // Pass 2 walks the keys in ascending order in chunks of 128: lane j computes e for key base+j,
 // lane 0 adds the denominators serially and lane d adds e*v[d] serially, so every sum keeps the
 // reference order.  The score is recomputed in pass 2 exactly as the reference does.
-// q: [tokens][1536]; cache of token b at k_cache + b*cache_stride (decode) or shared (prefill).
-// Decode key counts are clamped to max_keys (the cache rows the caller sized).
+// q: [tokens][1536]; cache of token b at k_cache + b*cache_stride.  Key counts are clamped to max_keys (the
+// cache rows the caller sized).
 // ---------------------------------------------------------------------------------------------
 __global__ void __launch_bounds__(128) attention_ordered_kernel(const float* __restrict__ q,
                                                                 const float* __restrict__ k_cache,
                                                                 const float* __restrict__ v_cache, size_t cache_stride,
-                                                                const int* __restrict__ pos, int max_keys, int prefill,
-                                                                int past, float* __restrict__ ctx) {
+                                                                const int* __restrict__ pos, int max_keys,
+                                                                float* __restrict__ ctx) {
   __shared__ float qs[QWEN_HEAD_DIM];
   __shared__ float es[128];
   __shared__ float red[128];
@@ -693,12 +691,12 @@ __global__ void __launch_bounds__(128) attention_ordered_kernel(const float* __r
   const int b = blockIdx.y;
   const int tid = threadIdx.x;
   const int kvh = h / QWEN_GROUPS;
-  const int n = prefill ? past + b + 1 : min(max(pos[b], 0) + 1, max_keys);
-  // Decode's (float)(1.0/sqrt(128.0)) and prefill's 0.08838834764831845f are the same float
-  // (bits 0x3db504f3; checked by tests/test_oracle_math.py).
+  const int n = min(max(pos[b], 0) + 1, max_keys);
+  // (float)(1.0/sqrt(128.0)) is this float, prefill's literal (bits 0x3db504f3; checked by
+  // tests/test_oracle_math.py).
   const float scaling = 0.08838834764831845f;
-  const float* kc = k_cache + (prefill ? 0 : (size_t)b * cache_stride) + kvh * QWEN_HEAD_DIM;
-  const float* vc = v_cache + (prefill ? 0 : (size_t)b * cache_stride) + kvh * QWEN_HEAD_DIM;
+  const float* kc = k_cache + (size_t)b * cache_stride + kvh * QWEN_HEAD_DIM;
+  const float* vc = v_cache + (size_t)b * cache_stride + kvh * QWEN_HEAD_DIM;
   qs[tid] = q[(size_t)b * QWEN_HIDDEN + h * QWEN_HEAD_DIM + tid];
   __syncthreads();
 
@@ -730,7 +728,7 @@ __global__ void __launch_bounds__(128) attention_ordered_kernel(const float* __r
       float score = 0.0f;
       for (int d = 0; d < QWEN_HEAD_DIM; ++d) score += qs[d] * kr[d];
       const float arg = score * scaling - m;
-      es[tid] = prefill ? approx_exp(arg) : glibc_expf(arg);
+      es[tid] = glibc_expf(arg);
     }
     __syncthreads();
     const int cnt = min(128, n - base);
@@ -747,14 +745,14 @@ __global__ void __launch_bounds__(128) attention_ordered_kernel(const float* __r
 }
 
 // ---------------------------------------------------------------------------------------------
-// The same attention in two launches, with the scores of all keys kept in between (the reference
+// The same attention, and the prefill's (prefill_attention_context_block, qwen_prefill_attention_kernel.cpp:
+// 204-289: keys 0..t, approx_exp), in two launches, with the scores of all keys kept in between (the reference
 // evaluates each score twice with the same operations, so keeping it gives the same bits).
 // scores: a block owns 64 keys of one KV head for QT query tokens; its key rows go through LDS once for
-// the six query heads (one wave each, lane = key, the 128 products of a score added in order).  577 keys of
-// one token: 5.7 + 8 us for the two launches, where one block per head that walked its keys alone took
-// 55 us.  ROPE
-// (one decode token): q is rotated on the way in, and the block that holds the new key's tile rotates
-// that key and appends the K and V rows, instead of a launch of its own.
+// the six query heads (one wave each, lane = key, the 128 products of a score added in order).  578 keys of
+// one token: 5.7 + 13.1 us for the two launches (traced in a resident step), where one block per head that
+// walked its keys alone took 55 us.  ROPE (one decode token): q is rotated on the way in, and the block that
+// holds the new key's tile rotates that key and appends the K and V rows, instead of a launch of its own.
 // scores[(token * 12 + head) * ld + key] = (q . k) * 1/sqrt(128).
 // grid = (ceil(tokens / QT), 2, key tiles), block = 384.  vec: the cache rows are 16-byte aligned.
 // ---------------------------------------------------------------------------------------------
@@ -967,15 +965,13 @@ void launch_chain(const OrdProject& a, int rows, hipStream_t st) {
   hipLaunchKernelGGL((project_chain_kernel<R, KC, PD, K, NORM, GU>), dim3(rows / R, a.tokens), dim3(256 + 4 * R), 0, st, a);
 }
 
-// Stagers pay wherever a CU has one block, and up to TT = 4 also beyond (their registers leave four waves
-// per SIMD; at TT = 8 and 16 they would cost the second block).
+// Stagers up to TT = 4 (their registers leave four waves per SIMD).  At TT = 8 and 16 they would cost the CU's
+// second block, and launch_mfma takes those forms for more blocks than CUs only.
 template <int TT, bool GU>
 void launch_mfma_tt(const OrdProject& a, int rows, hipStream_t st) {
-  const dim3 grid(rows / kMmRows, ceil_div(a.tokens, 4 * TT));
-  if (TT <= 4 || grid.x * grid.y <= 256)
-    hipLaunchKernelGGL((project_mfma_kernel<TT, GU, true>), grid, dim3(512), 0, st, a);
-  else
-    hipLaunchKernelGGL((project_mfma_kernel<TT, GU, false>), grid, dim3(256), 0, st, a);
+  constexpr bool kStagers = TT <= 4;
+  hipLaunchKernelGGL((project_mfma_kernel<TT, GU, kStagers>), dim3(rows / kMmRows, ceil_div(a.tokens, 4 * TT)),
+                     dim3(kStagers ? 512 : 256), 0, st, a);
 }
 
 template <bool GU>
@@ -1006,7 +1002,10 @@ void launch_mfma(const OrdProject& a, int rows, hipStream_t st) {
 
 }  // namespace
 
-// One block per 16 rows and token fits the chip at two blocks per CU: the chain kernel; more tokens: mfma.
+// The chain kernel up to five tokens of 1536 rows and four of 2048, mfma beyond.  A decode layer, chain against
+// mfma: o at 5 tokens 152 and 156 us, at 7 180 and 179, at 10 190 and 184; down at 3 tokens 136 and 163, at 5 151
+// and 174, at 6 182 and 179, at 10 220 and 184 (its 86 KB of LDS leave a CU one block, so three tokens and
+// more, 288 blocks and more, take a second round).
 bool ordered_chain_shape(int rows, int tokens) { return (long)rows / 16 * tokens <= 512; }
 
 void launch_project_ordered(const OrdProject& p, hipStream_t st) {
@@ -1058,10 +1057,9 @@ void launch_rope_table_prefill(float* rope, int first, int count, hipStream_t st
 }
 
 void launch_attention_ordered(const float* q, const float* k_cache, const float* v_cache, size_t cache_stride,
-                              const int* pos, int max_keys, int tokens, bool prefill, int past, float* ctx,
-                              hipStream_t st) {
+                              const int* pos, int max_keys, int tokens, float* ctx, hipStream_t st) {
   hipLaunchKernelGGL(attention_ordered_kernel, dim3(QWEN_Q_HEADS, tokens), dim3(128), 0, st, q, k_cache, v_cache,
-                     cache_stride, pos, max_keys, prefill ? 1 : 0, past, ctx);
+                     cache_stride, pos, max_keys, ctx);
 }
 
 namespace {

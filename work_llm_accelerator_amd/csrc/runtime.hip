@@ -190,10 +190,6 @@ DevLayer stage_layer(Arena& a, Staging& small, const HostLayer& h, hipStream_t s
 //   xn 1536, q 1536, k 256, v 256, ctx 1536 (attention);  pn 1536, s 8960 (MLP).
 // The attention and MLP executors each take their own part, so one token's layer needs the sum.
 namespace {
-size_t up64(size_t n) { return (n + 63u) & ~size_t(63u); }
-size_t decode_attention_floats(size_t T) { return 3u * up64(T * QWEN_HIDDEN) + 2u * up64(T * QWEN_KV_WIDTH); }
-size_t decode_mlp_floats(size_t T) { return up64(T * QWEN_HIDDEN) + up64(T * QWEN_INTERMEDIATE); }
-
 void carve_attention_part(DecodeWorkspace& w, float* p, size_t T) {
   auto take = [&](size_t n) {
     float* r = p;
@@ -227,10 +223,6 @@ size_t prefill_workspace_bytes(int tokens, int past) {
   const size_t T = (size_t)tokens;
   return (4u * T * QWEN_HIDDEN + T * QWEN_INTERMEDIATE + attention_ordered_scores(tokens, past + tokens)) *
              sizeof(float) + 6u * 256u;
-}
-
-size_t decode_workspace_floats(int tokens) {
-  return decode_attention_floats((size_t)tokens) + decode_mlp_floats((size_t)tokens);
 }
 
 DecodeWorkspace carve_decode_workspace(float* base, int tokens) {
@@ -320,7 +312,7 @@ void run_decode_attention_ws(const DevLayer& L, const float* x, const DecodeBatc
     }
     launch_attention_ordered_split(a, T, w.scores, st);
   } else {
-    launch_attention_ordered(w.q, b.k_cache, b.v_cache, b.cache_stride, b.pos, b.max_keys, T, false, 0, w.ctx, st);
+    launch_attention_ordered(w.q, b.k_cache, b.v_cache, b.cache_stride, b.pos, b.max_keys, T, w.ctx, st);
   }
   launch_project_ordered(row_project(w.ctx, T, QWEN_HIDDEN, L.ow, L.os, att, nullptr), st);
   QWEN_HIP(hipGetLastError());

@@ -177,7 +177,14 @@ struct DecodeWorkspace {
   float* scores = nullptr;
 };
 // Floats of a DecodeWorkspace of `tokens` rows, and its carve-up of `base` (each part 64-float aligned).
-size_t decode_workspace_floats(int tokens);
+constexpr size_t up64(size_t n) { return (n + 63u) & ~size_t(63u); }
+constexpr size_t decode_attention_floats(size_t T) {
+  return 3u * up64(T * QWEN_HIDDEN) + 2u * up64(T * QWEN_KV_WIDTH);
+}
+constexpr size_t decode_mlp_floats(size_t T) { return up64(T * QWEN_HIDDEN) + up64(T * QWEN_INTERMEDIATE); }
+constexpr size_t decode_workspace_floats(int tokens) {
+  return decode_attention_floats((size_t)tokens) + decode_mlp_floats((size_t)tokens);
+}
 DecodeWorkspace carve_decode_workspace(float* base, int tokens);
 void run_decode_attention_ws(const DevLayer& L, const float* x, const DecodeBatch& b, float* att,
                              const DecodeWorkspace& w, hipStream_t st);
