@@ -9,9 +9,9 @@
   group scales equals the int64 sum over groups exactly (a group dequantized with another group's
   scale, or rows of one group read into another, changes it).
 * Every kernel a FAST projection can take (the skinny decode GEMMs with one K group and with five
-  K splits, the direct-load kernel with its in-block K split, the pipelined GEMM with and without a
-  cross-block K split, the pipelined GEMM with two blocks per CU) accumulates the weight x activation
-  products exactly: with unit row scales and integer inputs whose largest magnitude is 32512 (so the
+  K splits, the direct-load kernel with its in-block K split, the pipelined GEMM in blocks of 32 and of
+  64 tokens, each with and without a cross-block K split) accumulates the weight x activation products
+  exactly: with unit row scales and integer inputs whose largest magnitude is 32512 (so the
   token scale is exactly 1 and the code is the input itself) and whose products stay below 2^24, the
   fp32 output is exactly the int64 product sum_k q(o, k) x(t, k), computed here with numpy.  A wrong
   nibble, limb, zero-point correction, K split or reduce order changes an integer and fails the
@@ -106,12 +106,18 @@ SHAPES = [
     (64, 8960, 1536, 0),    # skinny, 5 K splits, four token tiles (preloaded operands)
     (5, 8960, 1536, 1),     # direct-load kernel, in-block 4-way K split (no split workspace)
     (7, 1536, 1040, 0),     # direct-load kernel (out_dim not a multiple of 64)
-    (40, 1536, 1040, 0),    # pipelined 4-stage, cross-block K split over 12 blocks + reduce
-    (40, 1536, 1040, 1),    # pipelined 4-stage, no K split, partial row group
-    (150, 1536, 2048, 0),   # pipelined, 6 K splits, partial token tile
-    (150, 8960, 1536, 0),   # pipelined, 14 K splits
-    (300, 8960, 1536, 0),   # pipelined with two blocks per CU (no K split), partial token tile
-    (600, 1536, 2048, 0),   # pipelined with two blocks per CU
+    (40, 1536, 1040, 0),    # pipelined, 32-token blocks, cross-block K split over 12 blocks + reduce
+    (40, 1536, 1040, 1),    # 32-token blocks, no K split, partial row group
+    (150, 1536, 2048, 0),   # 32-token blocks, 3 K splits, partial token tile
+    (150, 8960, 1536, 0),   # 32-token blocks, 7 K splits
+    (300, 8960, 1536, 0),   # 32-token blocks, 2 K splits (each takes its own zero point off), partial token tile
+    (600, 1536, 2048, 0),   # 32-token blocks, no K split
+    (1030, 8960, 1536, 0),  # 64-token blocks, 5 K splits, partial token tile
+    (1030, 8960, 1536, 1),  # 64-token blocks, no K split
+    (1200, 8960, 1536, 0),  # 64-token blocks, 2 K splits
+    (1030, 1536, 1536, 0),  # 64-token blocks, no K split, the O shape
+    (2050, 8960, 1536, 0),  # 64-token blocks, no K split, the down shape of a long prefill
+    (8200, 1536, 1536, 0),  # more tokens than the split workspace has rows
 ]
 
 
@@ -128,7 +134,7 @@ def test_projection_integer_sums_exact(torch, lib, tokens, in_dim, out_dim, flag
     # exactness preconditions: the raw u = q + 8 sums of any K split (u <= 15) and the results stay
     # below 2^24 in magnitude, so every fp32 partial and sum is an exact integer
     assert np.all(15 * np.abs(X).sum(axis=1) < 2**24)
-    ref = X @ q.T  # [tokens][out] int64
+    ref = (X.astype(np.float64) @ q.T.astype(np.float64)).astype(np.int64)  # [tokens][out], exact below 2^53
     assert np.abs(ref).max() < 2**24
     wd = torch.from_numpy(packed).cuda()
     sw = torch.ones(out_dim, dtype=torch.float32, device="cuda")

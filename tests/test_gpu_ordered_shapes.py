@@ -1,7 +1,8 @@
 """ORDERED layers at the token counts where its projection kernels change form: chains of a few tokens,
-matrix-core products at 1, 2, 4, 8 and 16 tokens per wave, with remainders; key counts around the attention's
-64-key tiles; and row scales outside the range in which a weight is formed with one multiplication.  All
-bit for bit against the oracle (verification/real_host_top_backend.py runs the same layers on the host)."""
+matrix-core products at 1, 2, 4 and (gate/up) 8 tokens per wave, with remainders; key counts around the
+attention's 64-key tiles; and row scales outside the range in which a weight is formed with one multiplication.
+All bit for bit against the oracle (verification/real_host_top_backend.py runs the same layers on the host);
+the forms of 8 and 16 tokens per wave, which long prompts take, against chunks of the same prompt."""
 
 from __future__ import annotations
 
@@ -53,6 +54,33 @@ def test_prefill_tokens(layer, tokens):
     model.synchronize()
     for got, ref in ((hidden, out), (cache.k, kc), (cache.v, vc)):
         got = got.cpu().numpy().reshape(-1)
+        assert bits_equal(got, ref), first_mismatch(got, ref)
+    model.close()
+
+
+@pytest.mark.parametrize("tokens", [715, 2003])
+def test_prefill_in_chunks(layer, tokens):
+    """715 tokens: 8 a wave for q/k/v, 16 for gate/up; 2003: 16 for every projection.  In chunks of 128 all
+    run at 4 (each chunk's last tokens at fewer), which the oracle is compared with above."""
+    import torch
+
+    from work_llm_accelerator_amd.model import FLAG_NO_BF16_ROUND, MODE_ORDERED, KvCache
+
+    print(f"ordered prefill of {tokens} tokens, whole and in chunks", flush=True)
+    x = torch.from_numpy(random_hidden(920 + tokens, tokens).reshape(1, tokens, HIDDEN)).cuda()
+    model = model_of(layer)
+    whole, parts = KvCache.allocate(1, 1, tokens), KvCache.allocate(1, 1, tokens)
+    out = x.clone()
+    model.prefill(MODE_ORDERED | FLAG_NO_BF16_ROUND, out, whole)
+    model.synchronize()
+    for past in range(0, tokens, 128):
+        chunk = x[:, past:past + 128].clone()
+        model.prefill(MODE_ORDERED | FLAG_NO_BF16_ROUND, chunk, parts, past=past)
+        model.synchronize()
+        got, ref = out[0, past:past + 128].cpu().numpy().reshape(-1), chunk.cpu().numpy().reshape(-1)
+        assert bits_equal(got, ref), (past, first_mismatch(got, ref))
+    for got, ref in ((whole.k, parts.k), (whole.v, parts.v)):
+        got, ref = got.cpu().numpy().reshape(-1), ref.cpu().numpy().reshape(-1)
         assert bits_equal(got, ref), first_mismatch(got, ref)
     model.close()
 
