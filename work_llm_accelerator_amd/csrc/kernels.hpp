@@ -138,8 +138,6 @@ struct GemmArgs {
   int8_t* xq_out;
   float* sx_out;
   int* sums_out;
-  const int* zero_sums; // kFuseNormQuant, O of at most 64 tokens: optional zeros [tokens][2]; given, the
-                        // partial is the finished value (zero point off before its rounding, a prefill's)
   int defer_reduce;     // kFuseNormQuant, one token: write the partials only; the next projection's
                         // blocks finish the row (launch_gemm_i8_pre)
   int seq_len, past;    // kFuseRopePrefill (with rope, k_cache, v_cache, seq_stride, limit)

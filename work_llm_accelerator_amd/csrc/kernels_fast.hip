@@ -1132,10 +1132,14 @@ struct NoIssue {
   __device__ void operator()() const {}
 };
 
-// Elementwise pieces of the reduce step: the split sum plus zero-point correction (EXACT: the exact sum
+// What the partials of a reduce step hold: scaled fp32 sums with the zero point inside (the skinny and direct-load
+// kernels); the pipelined GEMM's int32 sums, all of which fit int32 with their zero point together (in_dim at most
+// kIntPartK), or only those of two of five splits, or of three of seven or more; or one split's finished value.
+constexpr int kPartScaled = 0, kExactNarrow = 1, kExactWide = 2, kPartFinished = 3;
+// Elementwise pieces of the reduce step: the split sum plus zero-point correction (exact forms: the exact sum
 // times the token's scale `corr` and the row scale), residual or bias, optional y_raw / y stores and bf16
 // rounding of elements row0 .. row0 + 3; the sum of squares of four elements in double; the RMSNorm scaling.
-template <int EPI, bool EXACT = false>
+template <int EPI, int FORM = kPartScaled>
 __device__ __forceinline__ float4 rnq_combine(const GemmArgs& a, int tok, int row0, float4 acc, float4 sw, float4 ad,
                                               double corr, bool write_y) {
   const float s4[4] = {sw.x, sw.y, sw.z, sw.w};
@@ -1144,7 +1148,9 @@ __device__ __forceinline__ float4 rnq_combine(const GemmArgs& a, int tok, int ro
   float out[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const float val = EXACT ? p4[q] * (float)corr * s4[q] : p4[q] + (float)(corr * (double)s4[q]);
+    const float val = FORM == kPartFinished ? p4[q]
+                      : FORM != kPartScaled ? p4[q] * (float)corr * s4[q]
+                                            : p4[q] + (float)(corr * (double)s4[q]);
     out[q] = EPI == kEpiResidual ? d4[q] + val : val + d4[q];
   }
   if (EPI == kEpiResidual && a.y_raw && write_y)
@@ -1188,11 +1194,8 @@ template <int EPI, class Issue = NoIssue>
 __device__ __forceinline__ void reduce_norm_quant_row(const GemmArgs& a, int splits, int tok, int8_t* xq_row,
                                                       int chunk_stride, float* sx_out, int* sums_out, bool write_y,
                                                       Issue&& issue = Issue{});
-// The partials of the pipelined GEMM: the sum of all splits fits int32 with its zero point (in_dim at most
-// kIntPartK), or only that of two of five splits, or of three of seven or more.
-constexpr int kExactNarrow = 1, kExactWide = 2;
 static_assert(kMaxQuantRow / 5 * 2 <= kIntPartK && kMaxQuantRow / 7 * 3 <= kIntPartK, "int32 groups of splits");
-template <int EPI, int ZB, class Issue, int W = 1, bool HOT = false, int EXACT = 0>
+template <int EPI, int ZB, class Issue, int W = 1, bool HOT = false, int FORM = kPartScaled>
 __device__ __forceinline__ void reduce_norm_quant_row_zb(const GemmArgs& a, int splits, int tok, int8_t* xq_row,
                                                          int chunk_stride, float* sx_out, int* sums_out, bool write_y,
                                                          Issue&& issue, const HotArgs& hot = HotArgs{});
@@ -2737,7 +2740,7 @@ __global__ void __launch_bounds__(256) reduce_norm_quant_kernel(GemmArgs a, int 
 // bias or a stand-in, p2 row scales, p3 norm weights or a stand-in, p4 limb sums, p5 scales, n0 the
 // token count), the flags read from `a` after the loads are issued; the outputs are the token's row
 // of a.xq_out (chunk_stride 256), a.sx_out and a.sums_out, whatever xq_row, sx_out and sums_out say.
-template <int EPI, int ZB, class Issue, int W, bool HOT, int EXACT>
+template <int EPI, int ZB, class Issue, int W, bool HOT, int FORM>
 __device__ __forceinline__ void reduce_norm_quant_row_zb(const GemmArgs& a, int splits, int tok, int8_t* xq_row,
                                                          int chunk_stride, float* sx_out, int* sums_out, bool write_y,
                                                          Issue&& issue, const HotArgs& hot) {
@@ -2776,9 +2779,9 @@ __device__ __forceinline__ void reduce_norm_quant_row_zb(const GemmArgs& a, int 
     ad[j] = r4[LS * j];
     wn[j] = w4[LS * j];
   }
-  // split sums in z order (EXACT: in integers, of groups whose sum fits int32, kExactNarrow: of all; one split,
-  // ZB = 1, holds the finished sum)
-  constexpr bool kInt = EXACT != 0 && ZB > 1, kWide = EXACT == kExactWide;
+  // split sums in z order (exact forms: in integers, of groups whose sum fits int32, kExactNarrow: of all; one
+  // split, ZB = 1, holds the exact sum in fp32)
+  constexpr bool kInt = (FORM == kExactNarrow || FORM == kExactWide) && ZB > 1, kWide = FORM == kExactWide;
   constexpr int kGroup = kWide ? (HOT ? 2 : 3) : ZB;
   long long tot[kInt ? NV : 1][4];
 #pragma unroll
@@ -2891,11 +2894,11 @@ __device__ __forceinline__ void reduce_norm_quant_row_zb(const GemmArgs& a, int 
                            exact_sum(tot[j][3] - zero));
   }
   const double corr =
-      EXACT ? (double)sx_tok : -8.0 * (256.0 * (double)sum_h + (double)sum_l) * (double)sx_tok;
+      FORM != kPartScaled ? (double)sx_tok : -8.0 * (256.0 * (double)sum_h + (double)sum_l) * (double)sx_tok;
   float4 v[NV];
 #pragma unroll
   for (int j = 0; j < NV; ++j)
-    v[j] = rnq_combine<EPI, EXACT != 0>(a, tok, 4 * (lane + LS * j), acc[j], sw[j], ad[j], corr, write_y);
+    v[j] = rnq_combine<EPI, FORM>(a, tok, 4 * (lane + LS * j), acc[j], sw[j], ad[j], corr, write_y);
   // RMSNorm (norm_quant_row's arithmetic, wave reductions)
   if (a.norm == kNormDecode) {
     double ss = 0.0;
@@ -3135,22 +3138,22 @@ __device__ __forceinline__ void reduce_norm_quant_row(const GemmArgs& a, int spl
 // grid = tokens, block = 128 (two waves per row: half the per-lane work of the one-wave form, three
 // LDS exchanges); the values equal the one-wave form's except the norm's sum of squares, added in
 // another order.
-template <int EPI, int EXACT>
+template <int EPI, int FORM>
 __global__ void __launch_bounds__(128) reduce_norm_quant_pair_kernel(GemmArgs a, int splits) {
   touch_kernargs<kernarg_bytes<GemmArgs, int>()>();
   const int tok = blockIdx.x;
   int8_t* xq_row = a.xq_out + (size_t)tok * (2 * QWEN_HIDDEN);
   if (splits == 1)
-    reduce_norm_quant_row_zb<EPI, 1, NoIssue, 2, false, EXACT>(a, splits, tok, xq_row, 256, a.sx_out + tok,
+    reduce_norm_quant_row_zb<EPI, 1, NoIssue, 2, false, FORM>(a, splits, tok, xq_row, 256, a.sx_out + tok,
                                                                a.sums_out + 2 * tok, true, NoIssue{});
   else
-    reduce_norm_quant_row_zb<EPI, EXACT != 0 ? 7 : 5, NoIssue, 2, false, EXACT>(a, splits, tok, xq_row, 256, a.sx_out + tok,
-                                                               a.sums_out + 2 * tok, true, NoIssue{});
+    reduce_norm_quant_row_zb<EPI, FORM != kPartScaled ? 7 : 5, NoIssue, 2, false, FORM>(
+        a, splits, tok, xq_row, 256, a.sx_out + tok, a.sums_out + 2 * tok, true, NoIssue{});
 }
 
 // The same with the first loads' operands preloaded (HotArgs of reduce_norm_quant_row_zb), residual
 // rows 1536 floats apart.
-template <int EPI, int EXACT>
+template <int EPI, int FORM>
 __global__ void __launch_bounds__(128) reduce_norm_quant_pair_hot_kernel(const void* p0, const void* p1, const void* p2,
                                                                          const void* p3, const void* p4, const void* p5,
                                                                          int tokens, int splits, GemmArgs a) {
@@ -3160,11 +3163,11 @@ __global__ void __launch_bounds__(128) reduce_norm_quant_pair_hot_kernel(const v
   auto issue = [&]() { kernarg_lines_wait(klines); };
   const int tok = blockIdx.x;
   // (the outputs are addressed inside, once the loads are issued)
-  if (splits == 1)
-    reduce_norm_quant_row_zb<EPI, 1, decltype(issue)&, 2, true, EXACT>(a, splits, tok, nullptr, 256, nullptr, nullptr,
+  if (FORM == kPartFinished || splits == 1)
+    reduce_norm_quant_row_zb<EPI, 1, decltype(issue)&, 2, true, FORM>(a, splits, tok, nullptr, 256, nullptr, nullptr,
                                                                        true, issue, hot);
   else
-    reduce_norm_quant_row_zb<EPI, 5, decltype(issue)&, 2, true, EXACT>(a, splits, tok, nullptr, 256, nullptr, nullptr,
+    reduce_norm_quant_row_zb<EPI, 5, decltype(issue)&, 2, true, FORM>(a, splits, tok, nullptr, 256, nullptr, nullptr,
                                                                        true, issue, hot);
 }
 
@@ -3887,31 +3890,37 @@ static void launch_gemm_t(const GemmArgs& a, hipStream_t st) {
 }
 
 // The reduce step after a GEMM that wrote partials (EXACT: the pipelined GEMM's): plain (bias / residual
-// epilogue) or fused.
+// epilogue) or fused with the next norm and quantization.
+template <int EPI, int FORM>
+static void launch_reduce_norm(const GemmArgs& a, int splits, hipStream_t st) {
+  if (a.out_dim == QWEN_HIDDEN && splits <= 5 && (EPI != kEpiResidual || a.resid_stride == QWEN_HIDDEN)) {
+    // the first loads' operands preloaded (an absent bias or norm weight read from the row scales)
+    const void* add = EPI == kEpiResidual ? (const void*)a.resid : a.bias ? (const void*)a.bias : a.sw;
+    const void* nw = a.norm != kNormNone ? (const void*)a.norm_w : a.sw;
+    hipLaunchKernelGGL((reduce_norm_quant_pair_hot_kernel<EPI, FORM>), dim3(a.tokens), dim3(128), 0, st,
+                       (const void*)a.part, add, (const void*)a.sw, nw, (const void*)a.sums, (const void*)a.sx, a.tokens,
+                       splits, a);
+    return;
+  }
+  if constexpr (FORM == kPartFinished) {
+    throw std::runtime_error("finished partials: one split of a 1536-wide projection only");
+  } else {
+    if (a.out_dim == QWEN_HIDDEN)
+      hipLaunchKernelGGL((reduce_norm_quant_pair_kernel<EPI, FORM>), dim3(a.tokens), dim3(128), 0, st, a, splits);
+    else
+      hipLaunchKernelGGL((reduce_norm_quant_kernel<EPI, FORM != kPartScaled>), dim3(a.tokens), dim3(256), 0, st, a,
+                         splits);
+  }
+}
 template <int EPI, bool EXACT = false>
 static void launch_reduce(const GemmArgs& a, int splits, hipStream_t st) {
   if (a.fuse == kFuseNormQuant) {
-    auto go = [&](auto form) {
-      constexpr int kForm = decltype(form)::value;
-      if (a.out_dim == QWEN_HIDDEN && splits <= 5 && (EPI != kEpiResidual || a.resid_stride == QWEN_HIDDEN)) {
-        // the first loads' operands preloaded (an absent bias or norm weight read from the row scales)
-        const void* add = EPI == kEpiResidual ? (const void*)a.resid : a.bias ? (const void*)a.bias : a.sw;
-        const void* nw = a.norm != kNormNone ? (const void*)a.norm_w : a.sw;
-        hipLaunchKernelGGL((reduce_norm_quant_pair_hot_kernel<EPI, kForm>), dim3(a.tokens), dim3(128), 0, st,
-                           (const void*)a.part, add, (const void*)a.sw, nw, (const void*)a.sums, (const void*)a.sx,
-                           a.tokens, splits, a);
-      } else if (a.out_dim == QWEN_HIDDEN) {
-        hipLaunchKernelGGL((reduce_norm_quant_pair_kernel<EPI, kForm>), dim3(a.tokens), dim3(128), 0, st, a, splits);
-      } else {
-        hipLaunchKernelGGL((reduce_norm_quant_kernel<EPI, EXACT>), dim3(a.tokens), dim3(256), 0, st, a, splits);
-      }
-    };
     if (!EXACT)
-      go(std::integral_constant<int, 0>{});
+      launch_reduce_norm<EPI, kPartScaled>(a, splits, st);
     else if (a.in_dim <= kIntPartK)
-      go(std::integral_constant<int, EXACT ? kExactNarrow : 0>{});
+      launch_reduce_norm<EPI, EXACT ? kExactNarrow : kPartScaled>(a, splits, st);
     else
-      go(std::integral_constant<int, EXACT ? kExactWide : 0>{});
+      launch_reduce_norm<EPI, EXACT ? kExactWide : kPartScaled>(a, splits, st);
   } else {
     const size_t quads = (size_t)a.tokens * (a.out_dim / 4);
     hipLaunchKernelGGL((gemm_splitk_reduce_kernel<EPI, EXACT>), dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, a,
@@ -4014,14 +4023,13 @@ static bool launch_skinny(const GemmArgs& a, hipStream_t st) {
     }
     if (!DUAL && a.fuse != kFuseNone && !a.part) return false;
     if constexpr (!DUAL && EPI == kEpiStore) {
-      if (a.fuse == kFuseNormQuant && a.zero_sums && a.out_dim == QWEN_HIDDEN) {  // finished partials
+      // a prefill's O: the finished value as the partial (a decode batch's holds its zero point, as ever)
+      if (a.fuse == kFuseNormQuant && a.norm == kNormPrefill && a.out_dim == QWEN_HIDDEN) {
         if (a.tokens > 16)
           launch_skinny_t<1, false, EPI, 12, false, 2, false, false, true>(a, row_tiles / 4, 1, st);
         else
           launch_skinny_t<1, false, EPI, 12, false, 1, false, false, true>(a, row_tiles / 4, 1, st);
-        GemmArgs r = a;
-        r.sums = a.zero_sums;
-        launch_reduce<EPI>(r, 1, st);
+        launch_reduce_norm<EPI, kPartFinished>(a, 1, st);
         return true;
       }
     }
@@ -4062,17 +4070,21 @@ static int device_cus() {
 
 // K splits of the two-blocks-per-CU pipelined GEMM with blocks of `tok` tokens and `tiles` row tiles: the least
 // of the time of its rounds (`alone` us per K chunk of a block alone on its CU, `pair` of two) and of the
-// partials' write and read, 2 us for the reduce launch where the call has none anyway.
+// partials' write and read at 4.5 TB/s, 2 us for the reduce launch where the call has none anyway.  What does not
+// depend on the split, about 3 us a launch, is left out.  Traced (down, 70 chunks): blocks of 32 tokens (0.5, 0.7)
+// 18.2 us at 512 tokens (960 blocks of 14 chunks) and 10.2 at 150 (420 of 10); of 64 tokens (0.9, 1.64) 65 us at
+// 1700 (162 blocks of 70), 39 at 1200 (228 of 35) and 40 at 1030 (510 of 14); two on a CU without partials are
+// faster than that (101 us at 4096 tokens, 384 blocks of 70).
 static int pipe_splits(const GemmArgs& a, int tok, int tiles, double alone, double pair) {
   if (!a.part || a.out_dim > QWEN_QKV_ROWS) return 1;
-  const int nkc = a.in_dim / kKChunk;
+  const int nkc = a.in_dim / kKChunk, cus = device_cus();
   const int blocks = (a.tokens + tok - 1) / tok * ((a.out_dim / 16 + tiles - 1) / tiles);
   int best = 1;
   double cost = 0.0;
   for (int s = 1; s <= kMaxSplits; ++s) {
     if (nkc % s != 0 || (s > 1 && s * a.tokens > kSplitRows)) continue;
     const int n = blocks * s;
-    const double rounds = n <= 256 ? alone : pair * ((n + 511) / 512);
+    const double rounds = n <= cus ? alone : pair * ((n + 2 * cus - 1) / (2 * cus));
     const double c = rounds * (nkc / s) + (s > 1 || a.fuse != kFuseNone ? s * (double)a.tokens * a.out_dim * 8.0 / 4.5e6 : 0.0) +
                      (s > 1 && a.fuse == kFuseNone ? 2.0 : 0.0);
     if (s == 1 || c < cost) {
@@ -4117,7 +4129,7 @@ static void launch_gemm_epi(const GemmArgs& a, hipStream_t st) {
         throw std::runtime_error("RoPE epilogue: more than 64 tokens of the [q | k | v] projection");
       // one head and 32 tokens per block while two-head blocks of 64 tokens (8 per 64 tokens) do not fill the CUs
       // (512 tokens: 17.2 us; one head of 64 tokens 12.0 us, of 32 tokens 8.9 us)
-      const bool few = (a.tokens + 63) / 64 * 8 <= 256;
+      const bool few = (a.tokens + 63) / 64 * 8 <= device_cus();
       if (a.fuse == kFuseQkvRope) {
         if (few)
           launch_gemm_pipe_t<2, 2, 2, EPI, DUAL, 1, 2, false, true, true>(a, 1, st);

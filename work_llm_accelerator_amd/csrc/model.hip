@@ -454,7 +454,6 @@ struct qwen_hip_model {
     fn.xq_out = w.xq;
     fn.sx_out = w.sx;
     fn.sums_out = w.sums;
-    if (grouped) fn.zero_sums = w.zero_sums;
     for (int i = 0; i < count; ++i) {
       const FastLayer& f = fast[first + i];
       float* kc = kc0 + (size_t)i * ls;
